@@ -31,6 +31,7 @@
 //   gqa_combine_kernel    rescales the splits to the common maximum and normalises
 //   gqa_attention_kernel  any other head_dim: one workgroup per unit, keys strided over
 //                         the threads
+// Prompts of 128 keys or more run on gqa_split.h's kernels when the caller gives a workspace.
 #pragma once
 #include "decoder_ops.h"
 

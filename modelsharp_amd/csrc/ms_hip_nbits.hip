@@ -50,6 +50,7 @@
 #include "generic_nbits.h"
 #include "mfma_general.h"
 #include "w4a8.h"
+#include "gqa_split.h"
 #include "gqa.h"
 #include "mfma_w4.h"
 #include "mfma_w4_pipe.h"
@@ -2945,6 +2946,7 @@ struct GqaPlan {
     int G = 0;          // lanes per row of gqa_rows_kernel<G>, 0: gqa_attention_kernel
     bool grouped = false;   // gqa_group_kernel<D> (every query head of a kv group per workgroup)
     bool flash = false;     // gqa_flash_kernel<D> (prefill on the fp32 matrix cores)
+    int split_waves = 0;    // gqa_split_kernel<D, split_waves> (prefill on fp16 halves), 0: another
     int splits = 1;
     size_t lds = 0;
     int64_t ws_bytes = 0;
@@ -2952,10 +2954,41 @@ struct GqaPlan {
 
 constexpr size_t kGqaMaxLds = 160 * 1024;
 
-GqaPlan gqa_plan(const ms_hip_gqa_desc& d, int64_t ws_avail)
+// Prompts on the fp16 matrix cores (gqa_split.h): more than 8 queries, a workspace for the
+// keys' and values' halves, and a positive scale that keeps finite scores finite.
+// From 128 keys on (192 with head_dim 64, whose chunks are half as long): the conversion's
+// launch and the longer prologue cost about 5 us, which the chunks repay from there (28 heads
+// of 128, measured before -> with it: 96 keys 25.8 -> 25.9, 128 keys 30.9 -> 26.5, 200 keys
+// 37.3 -> 30.8, 512 keys 65.5 -> 41.3 us; head_dim 64: 8 heads, 64 keys 15.3 -> 17.1, 160 keys
+// 20.0 -> 19.5, 14 heads, 134 keys 18.8 -> 20.9, 612 keys 45.0 -> 30.5 us). A window that
+// shows the queries less than half of the keys does not repay converting all of them.
+// head_dim 256 stays with gqa_rows_kernel, whose sums are closer to 64 bits than these.
+bool gqa_split_fits(const ms_hip_gqa_desc& d)
+{
+    const int D = d.head_dim;
+    const int64_t total = (int64_t)d.past_seq + d.kv_seq;
+    const int64_t visible = d.local_window_size >= 0 ? std::min(total, (int64_t)d.local_window_size + d.q_seq) : total;
+    return d.q_seq > 8 && (D == 64 || D == 96 || D == 128) && d.batch > 0 && visible >= (D == 64 ? 192 : 128) && total <= 2 * visible &&
+           d.scale >= 0.0f && d.scale <= 65536.0f && gqa_split_chunks(total) * (int64_t)(512 * D) < kPipeFar &&
+           (int64_t)d.batch * d.kv_num_heads * gqa_split_chunks(total) < (1 << 30);
+}
+
+GqaPlan gqa_plan(const ms_hip_gqa_desc& d, int64_t ws_avail, bool split_ok = true)
 {
     GqaPlan pl;
     const int D = d.head_dim;
+    if (split_ok && gqa_split_fits(d)) {
+        const int64_t ws = gqa_split_ws_bytes((int64_t)d.batch * d.kv_num_heads, (int64_t)d.past_seq + d.kv_seq, D);
+        if (ws_avail < 0 || ws <= ws_avail) {
+            // 128 queries per workgroup while that still gives every CU one, else 64 (a block of
+            // 64 halves a short launch's waves, and its idle CUs)
+            const int64_t wg = (int64_t)d.batch * d.num_heads * ((d.q_seq + 127) / 128);
+            pl.split_waves = wg >= 256 ? 4 : 2;
+            pl.lds = (size_t)1024 * D;
+            pl.ws_bytes = ws;
+            return pl;
+        }
+    }
     const int64_t total = (int64_t)d.past_seq + d.kv_seq;
     const int64_t units = (int64_t)d.batch * d.num_heads * d.q_seq;
     const int grp = d.kv_num_heads > 0 ? d.num_heads / d.kv_num_heads : 0;
@@ -3006,6 +3039,32 @@ GqaPlan gqa_plan(const ms_hip_gqa_desc& d, int64_t ws_avail)
     return pl;
 }
 
+template <int D, int NW>
+int launch_gqa_split_attention(const GqaArgs& p, const GqaPlan& pl, const GqaSplitWs& w, hipStream_t s)
+{
+    const int64_t grid = gqa_split_grid(p.B * p.kvH, p.H / p.kvH, (p.Sq + 32 * NW - 1) / (32 * NW));
+    if (pl.lds >= 64 * 1024)   // with the kernel's few static bytes above 64 KB
+        MS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(gqa_split_kernel<D, NW>),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.lds));
+    hipLaunchKernelGGL((gqa_split_kernel<D, NW>), dim3((unsigned)grid), dim3(128 * NW), pl.lds, s, p, w);
+    MS_HIP_CHECK(hipGetLastError());
+    return MS_HIP_OK;
+}
+
+template <int D>
+int launch_gqa_split(const GqaArgs& p, const GqaPlan& pl, void* workspace, hipStream_t s)
+{
+    const int units = p.B * p.kvH, nch = gqa_split_chunks(p.total);
+    GqaSplitWs w;
+    w.img = static_cast<uint8_t*>(workspace);
+    w.exps = reinterpret_cast<int*>(w.img + (int64_t)units * nch * (512 * D));
+    w.nch = nch;
+    hipLaunchKernelGGL(gqa_split_kv_kernel<D>, dim3((unsigned)(2 * units * nch)), dim3(256), 0, s, p, w);
+    MS_HIP_CHECK(hipGetLastError());
+    return pl.split_waves == 4 ? launch_gqa_split_attention<D, 4>(p, pl, w, s)
+                               : launch_gqa_split_attention<D, 2>(p, pl, w, s);
+}
+
 }  // namespace
 
 extern "C" {
@@ -3035,7 +3094,7 @@ int ms_hip_gqa_check(const ms_hip_gqa_desc* d)
     if (d->do_rotary && (d->cos_rows <= 0 || d->cos_cols <= 0))
         return fail(MS_HIP_ERR_INVALID,
                     "GroupQueryAttention do_rotary=1 requires cos_cache (input 7) and sin_cache (input 8).");
-    const int64_t lds = (int64_t)gqa_plan(*d, -1).lds;
+    const int64_t lds = (int64_t)gqa_plan(*d, -1, false).lds;
     if (lds > (int64_t)kGqaMaxLds)
         return fail(MS_HIP_ERR_UNSUPPORTED,
                     "[ms_hip] GroupQueryAttention keeps a unit's scores in LDS: total sequence %lld with head_dim %d "
@@ -3108,7 +3167,16 @@ int ms_hip_gqa(const ms_hip_gqa_desc* d, const float* dQ, const float* dK, const
         hipLaunchKernelGGL(gqa_copy_past_kernel, dim3(elementwise_grid(n)), dim3(256), 0, s, p);
         MS_HIP_CHECK(hipGetLastError());
     }
-    const GqaPlan plan = p.Sq > 0 ? gqa_plan(*d, dWorkspace && !misaligned4(dWorkspace) ? workspace_bytes : 0) : GqaPlan{};
+    const GqaPlan plan = p.Sq > 0 ? gqa_plan(*d, dWorkspace && !misaligned4(dWorkspace) ? workspace_bytes : 0,
+                                             (reinterpret_cast<uintptr_t>(dWorkspace) & 15) == 0)
+                                  : GqaPlan{};
+    if (plan.split_waves) {
+        switch (p.D) {
+            case 64: return launch_gqa_split<64>(p, plan, dWorkspace, s);
+            case 96: return launch_gqa_split<96>(p, plan, dWorkspace, s);
+            default: return launch_gqa_split<128>(p, plan, dWorkspace, s);
+        }
+    }
     if (p.Skv > 0 && !plan.grouped) {   // the grouped kernel writes the new rows itself
         const int threads = std::min(256, ((p.D + 63) / 64) * 64);
         hipLaunchKernelGGL(gqa_append_kernel, dim3((unsigned)(p.B * p.Skv * p.kvH)), dim3(threads), 0, s, p);

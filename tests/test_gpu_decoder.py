@@ -391,6 +391,53 @@ def test_gqa_flash_cases(gpu, case):
               f"flash seed {case['seed']}")
 
 
+# The same operator with a workspace: gqa_split_kernel (fp16 halves), every head_dim it takes,
+# ragged query blocks (32 queries a wave, 64 or 128 a workgroup) and key chunks (64), and
+# every way its work is dealt to the XCDs (B * KH dividing 8, a multiple of 8, neither).
+SPLIT_CASES = FLASH_CASES + [
+    dict(seed=221, B=1, Sq=9, H=4, KH=1, D=96, past=120, cos_rows=160),
+    dict(seed=222, B=1, Sq=65, H=6, KH=3, D=96, past=63, cos_rows=160, packed=True),
+    dict(seed=223, B=2, Sq=33, H=4, KH=2, D=96, past=131, cos_rows=180, cos_cols=21),   # an odd rotary half
+    dict(seed=224, B=2, Sq=230, H=16, KH=8, D=64, past=0, cos_rows=230),
+    dict(seed=225, B=1, Sq=300, H=64, KH=4, D=96, past=7, cos_rows=320, interleaved=True),
+    dict(seed=226, B=3, Sq=194, H=2, KH=1, D=64, past=0, window=40, cos_rows=194),
+    dict(seed=227, B=2, Sq=192, H=64, KH=16, D=64, past=1, seqlens=[5, 192], cos_rows=200),
+    dict(seed=229, B=2, Sq=70, H=4, KH=2, D=128, past=64, window=90, kv_seq=71, cos_rows=160),
+]
+
+
+@pytest.mark.parametrize("case", SPLIT_CASES, ids=lambda c: f"seed{c['seed']}")
+def test_gqa_split_cases(gpu, case):
+    d, q, k, v, pk, pv, sl, cos, sin = make_case(**case)
+    ref, rk, rv = oracle.gqa(d, q, k, v, pk, pv, sl, cos, sin)
+    check_gqa(*run_device_gqa(d, q, k, v, pk, pv, sl, cos, sin, capacity=d.past_seq + d.kv_seq + 5, workspace=True),
+              ref, rk, rv, f"split seed {case['seed']}")
+
+
+@pytest.mark.parametrize("where,value", [("k", np.inf), ("k", -np.inf), ("k", np.nan), ("k", 3e18), ("k", 1e6),
+                                         ("k", 1e3), ("q", np.inf),
+                                         ("q", np.nan), ("q", 2e15), ("v", np.inf), ("v", np.nan), ("v", 3e38),
+                                         ("v", 1e6), ("v", 1e3), ("v", 1e-30)])
+def test_gqa_split_extreme_values(gpu, where, value):
+    """One value the fp16 halves cannot carry, or can only just: the rows that see it are the
+    oracle's (NaN where it is NaN), and rows before it are unaffected."""
+    d, q, k, v, pk, pv, sl, cos, sin = make_case(231, B=1, Sq=150, H=4, KH=2, D=128, past=0, rotary=False, cos_rows=8)
+    t = {"q": q, "k": k, "v": v}[where]
+    t[0, 70, 5] = value
+    if where == "v" and value == 1e-30:   # a chunk whose values are all tiny beside one of ordinary ones
+        t[0, 64:128] *= np.float32(value)
+    with np.errstate(all="ignore"):
+        ref, rk, rv = oracle.gqa(d, q, k, v, pk, pv, sl, cos, sin)
+        out, PK, PV = run_device_gqa(d, q, k, v, pk, pv, sl, cos, sin, workspace=True)
+        assert np.array_equal(PK, rk, equal_nan=True) and np.array_equal(PV, rv, equal_nan=True)
+        assert np.array_equal(np.isnan(out), np.isnan(ref)) and np.array_equal(np.isinf(out), np.isinf(ref))
+        # a row's bar is its own: rows with one huge value are not the others' measure
+        ok = np.isfinite(ref)
+        rows = np.abs(np.where(ok, ref, 0.0)).reshape(150 * 4, 128).max(axis=1, keepdims=True)
+        err = np.abs(np.where(ok, out - ref, 0.0)).reshape(150 * 4, 128)
+    assert np.all(err <= 1e-5 * rows)
+
+
 @pytest.mark.parametrize("workspace", [False, True], ids=["one_split", "key_splits"])
 @pytest.mark.parametrize("Sq,past,KH", [(1, 2047, 8), (1, 4095, 32), (128, 0, 8), (16, 300, 8)])
 def test_gqa_7b_shapes(gpu, Sq, past, KH, workspace):
