@@ -1599,40 +1599,79 @@ int enqueue_gemm(Weights& w, const float* dA, float* dY, int M, hipStream_t stre
 }
 
 // ---- W4A8 (the opt-in approximate product) --------------------------------------------------
-// Workspace of one call: activation codes [M][padK], their scales [M][nb] and the
-// transposed scales [nb][Mp], each 256-byte aligned.
+enum W4a8KernelId { kW8Gemv = 9, kW8Mfma = 10, kW8Generic = 11 };
+
+// The GEMM's dots are exact while a block's sum stays below 2^24.
+W4a8KernelId w4a8_kernel(const Weights& w, int M)
+{
+    if (w.bits == 4 && w.bs % 32 == 0) {
+        if (M <= 16) return kW8Gemv;
+        if ((int64_t)w.bs * 127 * 15 < (1 << 24)) return kW8Mfma;
+    }
+    return kW8Generic;
+}
+
+// Rows of A per workgroup of the GEMM, in units of 16: the least work on the fullest CU,
+// which runs ceil(workgroups / 256) of them; per 32-code step about 21 VALU instructions for
+// the weights' dequant and the loop, and per unit 12 / spb for the sums and 2 for what of the
+// MFMAs they do not cover.
+int w4a8_nf(const Weights& w, int M)
+{
+    int best = 2;
+    int64_t cost = INT64_MAX;
+    for (int nf : {8, 4, 2}) {
+        const int64_t wgs = (int64_t)((M + 16 * nf - 1) / (16 * nf)) * ((w.N + kW8BN - 1) / kW8BN);
+        const int spb = w.bs / 32;
+        const int64_t c = (wgs + device_cus() - 1) / device_cus() * ((12 + 2 * spb) * nf + 21 * spb);
+        if (c < cost) {
+            cost = c;
+            best = nf;
+        }
+    }
+    return best;
+}
+
+// Workspace of one call. The GEMM: the images of A (w4a8_stage_kernel). The others:
+// activation codes [M][padK] and, 256-byte aligned, their scales [M][nb].
 struct W4a8Layout {
-    int padK = 0, Mp = 0;
-    size_t sa_off = 0, sat_off = 0, total = 0;
+    int padK = 0, nf = 0, tiles_m = 0, G = 0;
+    size_t sa_off = 0, total = 0;
 };
 
 W4a8Layout w4a8_layout(const Weights& w, int M)
 {
     W4a8Layout L;
     L.padK = ((w.nb * w.bs + 31) / 32) * 32;
-    L.Mp = ((M + 3) / 4) * 4;
+    if (w4a8_kernel(w, M) == kW8Mfma) {
+        L.nf = w4a8_nf(w, M);
+        L.tiles_m = (M + 16 * L.nf - 1) / (16 * L.nf);
+        L.G = (L.padK / 32 + 3) / 4;
+        L.total = (size_t)L.tiles_m * L.G * w4a8_image_bytes(L.nf);
+        return L;
+    }
     L.sa_off = align256((size_t)M * L.padK);
-    L.sat_off = L.sa_off + align256((size_t)M * w.nb * sizeof(float));
-    L.total = L.sat_off + align256((size_t)w.nb * L.Mp * sizeof(float));
+    L.total = L.sa_off + align256((size_t)M * w.nb * sizeof(float));
     return L;
-}
-
-enum W4a8KernelId { kW8Gemv = 9, kW8Mfma = 10, kW8Generic = 11 };
-
-W4a8KernelId w4a8_kernel(const Weights& w, int M)
-{
-    if (w.bits == 4 && w.bs % 32 == 0) return M <= 16 ? kW8Gemv : kW8Mfma;
-    return kW8Generic;
 }
 
 int w4a8_grid(const Weights& w, int M, W4a8KernelId k)
 {
     if (k == kW8Gemv) return (w.N + kW8RowsPerWg - 1) / kW8RowsPerWg;
     if (k == kW8Mfma) {
-        const int tiles = ((M + kW8BM - 1) / kW8BM) * ((w.N + kW8BN - 1) / kW8BN);
+        const int tiles = w4a8_layout(w, M).tiles_m * ((w.N + kW8BN - 1) / kW8BN);
         return ((tiles + kXcds - 1) / kXcds) * kXcds;
     }
     return (int)(((int64_t)M * w.N + 255) / 256);
+}
+
+typedef void (*W8MfmaFn)(W4a8MfmaParams);
+template <int NF>
+W8MfmaFn w8_mfma_fn(int spb)
+{
+    return spb == 1       ? mfma_w4a8_kernel<NF, 1>
+           : spb == 2     ? mfma_w4a8_kernel<NF, 2>
+           : spb % 4 == 0 ? mfma_w4a8_kernel<NF, 4>
+                          : mfma_w4a8_kernel<NF, 0>;
 }
 
 typedef void (*W8GemvFn)(RawLayout, W4a8Args, float*);
@@ -1646,36 +1685,47 @@ constexpr auto kW8GemvTable = w8_gemv_table(std::make_index_sequence<16>{});
 int launch_w4a8(const Weights& w, const Ws& ws, const float* dA, float* dY, int M, hipStream_t stream)
 {
     const W4a8Layout Lw = w4a8_layout(w, M);
+    const RawLayout L = raw_layout(w);
+    const W4a8KernelId k = w4a8_kernel(w, M);
+    const int grid = w4a8_grid(w, M, k);
+    if (k == kW8Mfma) {
+        const int64_t threads = (int64_t)M * w.nb * 4;
+        hipLaunchKernelGGL(w4a8_stage_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, dA,
+                           ws.data, M, w.K, w.bs, w.nb, Lw.G, Lw.nf);
+        MS_HIP_CHECK(hipGetLastError());
+        W4a8MfmaParams p;
+        p.L = L;
+        p.img = ws.data;
+        p.y = dY;
+        p.M = M;
+        p.G = Lw.G;
+        p.tiles_m = Lw.tiles_m;
+        p.tiles_n = (w.N + kW8BN - 1) / kW8BN;
+        const int spb = w.bs / 32;
+        const W8MfmaFn fn = Lw.nf == 2 ? w8_mfma_fn<2>(spb) : Lw.nf == 4 ? w8_mfma_fn<4>(spb) : w8_mfma_fn<8>(spb);
+        const int lds = 2 * w4a8_image_bytes(Lw.nf);
+        if (lds > 64 * 1024)
+            MS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             lds));
+        hipLaunchKernelGGL(fn, dim3(grid), dim3(256), lds, stream, p);
+        MS_HIP_CHECK(hipGetLastError());
+        return MS_HIP_OK;
+    }
     int8_t* aq = reinterpret_cast<int8_t*>(ws.data);
     float* sa = reinterpret_cast<float*>(ws.data + Lw.sa_off);
-    float* sat = reinterpret_cast<float*>(ws.data + Lw.sat_off);
-    const int64_t threads = (int64_t)Lw.Mp * w.nb * 8;
+    const int64_t threads = (int64_t)M * w.nb * 8;
     hipLaunchKernelGGL(w4a8_quantize_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, dA, aq,
-                       sa, sat, M, Lw.Mp, w.K, w.bs, w.nb, Lw.padK);
+                       sa, M, w.K, w.bs, w.nb, Lw.padK);
     MS_HIP_CHECK(hipGetLastError());
     W4a8Args A;
     A.aq = aq;
     A.sa = sa;
-    A.sat = sat;
     A.M = M;
-    A.Mp = Lw.Mp;
     A.padK = Lw.padK;
-    const RawLayout L = raw_layout(w);
-    const W4a8KernelId k = w4a8_kernel(w, M);
-    const int grid = w4a8_grid(w, M, k);
-    if (k == kW8Gemv) {
+    if (k == kW8Gemv)
         hipLaunchKernelGGL(kW8GemvTable[M - 1], dim3(grid), dim3(256), 0, stream, L, A, dY);
-    } else if (k == kW8Mfma) {
-        W4a8MfmaParams p;
-        p.L = L;
-        p.A = A;
-        p.y = dY;
-        p.tiles_m = (M + kW8BM - 1) / kW8BM;
-        p.tiles_n = (w.N + kW8BN - 1) / kW8BN;
-        hipLaunchKernelGGL(mfma_w4a8_kernel, dim3(grid), dim3(256), 0, stream, p);
-    } else {
+    else
         hipLaunchKernelGGL(w4a8_generic_kernel, dim3(grid), dim3(256), 0, stream, L, A, dY);
-    }
     MS_HIP_CHECK(hipGetLastError());
     return MS_HIP_OK;
 }

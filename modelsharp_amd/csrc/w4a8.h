@@ -14,25 +14,20 @@
 // independent of the order of their terms, so the weights need no byte permutation.
 //
 // Kernels:
-//   w4a8_quantize_kernel   8 lanes per (row, block): aq [M][padK], s_a [M][nb] and its
-//                          transpose [nb][Mp] (Mp = M rounded up to 4, zero rows past M)
+//   w4a8_quantize_kernel   8 lanes per (row, block): aq [M][padK], s_a [M][nb]
 //   gemv_w4a8_kernel<M>    M <= 16, 4-bit codes, block size a multiple of 32: 16 lanes per
 //                          weight row, lane g takes blocks g, g + 16, ...; each round of 16
 //                          blocks leaves its 16 terms per row of A in LDS and lane m of the
 //                          row adds them, in block order, to row m's sum
-//   mfma_w4a8_kernel       M > 16, same formats: a 128 x 64 tile of Y per workgroup,
-//                          v_mfma_i32_32x32x32_i8 per 32 codes into an int32 block
-//                          accumulator, rescaled into the fp32 sum at each block's end
+//   w4a8_stage_kernel, mfma_w4a8_kernel   M > 16, same formats: block dots on the fp16
+//                          matrix cores (exact), rescaled into the fp32 sums at each block's end
 //   w4a8_generic_kernel    every other format (8-bit codes, any block size): one thread
 //                          per output, the definition above as written
 #pragma once
 #include "generic_nbits.h"
-#include "mfma_w4.h"
+#include "mfma_w4_pipe.h"
 
 namespace msnb {
-
-typedef int v4i_t __attribute__((ext_vector_type(4)));
-typedef int v16i_t __attribute__((ext_vector_type(16)));
 
 // Position of k in the nibble-ordered code row.
 __device__ __forceinline__ int w4a8_pos(int k)
@@ -44,24 +39,19 @@ __device__ __forceinline__ int w4a8_pos(int k)
 struct W4a8Args {
     const int8_t* aq;   // [M][padK] nibble order, zero past K
     const float* sa;    // [M][nb]
-    const float* sat;   // [nb][Mp]
-    int M, Mp, padK;
+    int M, padK;
 };
 
 // ---- activation quantizer (qgemm_w4a8.cpp:257-285) -----------------------------------------
 __global__ __launch_bounds__(256) void w4a8_quantize_kernel(const float* __restrict__ a, int8_t* __restrict__ aq,
-                                                            float* __restrict__ sa, float* __restrict__ sat, int M,
-                                                            int Mp, int K, int bs, int nb, int padK)
+                                                            float* __restrict__ sa, int M, int K, int bs, int nb,
+                                                            int padK)
 {
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int j = (int)(gid & 7);
-    const int64_t blk = gid >> 3;              // (row, block) id; rows M..Mp-1 only clear sat
-    if (blk >= (int64_t)Mp * nb) return;       // whole groups of 8 lanes leave together
+    const int64_t blk = gid >> 3;             // (row, block) id
+    if (blk >= (int64_t)M * nb) return;       // whole groups of 8 lanes leave together
     const int m = (int)(blk / nb), bk = (int)(blk - (int64_t)m * nb);
-    if (m >= M) {
-        if (j == 0) sat[(int64_t)bk * Mp + m] = 0.0f;
-        return;
-    }
     const int k0 = bk * bs;
     const int len = min(bs, K - k0);
     const float* arow = a + (int64_t)m * K + k0;
@@ -81,10 +71,7 @@ __global__ __launch_bounds__(256) void w4a8_quantize_kernel(const float* __restr
         }
         qrow[w4a8_pos(k0 + i)] = (int8_t)q;
     }
-    if (j == 0) {
-        sa[(int64_t)m * nb + bk] = s;
-        sat[(int64_t)bk * Mp + m] = s;
-    }
+    if (j == 0) sa[(int64_t)m * nb + bk] = s;
 }
 
 // Signed codes (code - zp, as int8 bytes) of 8 packed 4-bit codes: the even k, the odd k.
@@ -171,116 +158,253 @@ __global__ __launch_bounds__(256) void gemv_w4a8_kernel(RawLayout L, W4a8Args A,
     if (live && g < M) y[(int64_t)g * L.N + n] = acc;
 }
 
-// ---- prefill on the int8 matrix cores ---------------------------------------------------------
-constexpr int kW8BM = 128, kW8BN = 64;
+// ---- prefill on the matrix cores ----------------------------------------------------------------
+// The reference rounds three times per output and block ((s_a s_w), times the dot, added),
+// so the fp32 VALU bounds this product: 3 instructions per output and block, 28 us for
+// M=256, K=4096, N=11008 at bs=32. Everything else is arranged around them:
+//   * the block dot comes out of v_mfma_f32_16x16x32_f16 as fp32: the codes are fp16
+//     integers (|aq| <= 127, |wc| <= 15), their products and sums below 2^24 exact, so no
+//     conversion follows (the int8 MFMA needs one per output and block: a fourth instruction,
+//     against 5 more for the 8 weight codes of a lane, shared by 16 NF outputs);
+//   * a wave owns 16 weight rows and 16 NF rows of A: a lane dequantizes 8 codes per 32-code
+//     step (11 instructions) for 4 NF outputs. Weights never touch LDS: lane (n, s) loads the
+//     16 bytes of step 4 g + s of row n, and v_permlane swaps turn four steps' rows of lanes
+//     into the operands;
+//   * A is staged by w4a8_stage_kernel in LDS image order, one image per 4 steps with the
+//     block scales behind the codes, double-buffered through buffer->LDS loads issued a
+//     group ahead: one barrier per 128 k, no bank conflicts.
+// Workgroups of 4 waves take 64 weight rows; NF (2, 4 or 8) by launch size.
+// M=256, K=4096, N=11008, bs=32: 156 -> 80 us; M=128, K=11008, N=4096, bs=128: 254 -> 88 us;
+// M=17, K=4096, N=4096: 132 -> 50 us (against an int8 MFMA, a barrier per 32 codes and loads
+// that were not ahead). What is left above the VALU's time is the wait for each group's loads.
+constexpr int kW8BN = 64;
+constexpr int w4a8_image_bytes(int nf) { return 4608 * nf; }   // 4 steps: codes 4096, scales 256, padding
+
+// LDS image of rows [16 nf t, ...) and steps [4 g, 4 g + 4): codes at ((b nf + f) 64 + lane) 16
+// (step b, row 16 f + lane % 16, k = 8 (lane / 16) + [0, 8) in the order of dequant8_f16's
+// pairs), then the block's scale at 4096 nf + ((b 16 + row % 16) nf + f) 4.
+// Four lanes per (row, block): the max over the block by two lane exchanges, arithmetic of
+// w4a8_quantize_kernel. Rows past M are left as they are: no output depends on them.
+__global__ __launch_bounds__(256) void w4a8_stage_kernel(const float* __restrict__ a, uint8_t* __restrict__ img, int M,
+                                                         int K, int bs, int nb, int G, int nf)
+{
+    typedef float f4u_t __attribute__((ext_vector_type(4), aligned(4)));
+    const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int j = (int)(gid & 3);
+    const int64_t blk = gid >> 2;
+    if (blk >= (int64_t)M * nb) return;   // whole groups of 4 lanes leave together
+    const int m = (int)(blk / nb), bk = (int)(blk - (int64_t)m * nb);
+    const int k0 = bk * bs, len = min(bs, K - k0);
+    const float* arow = a + (int64_t)m * K + k0;
+    auto load8 = [&](int i, float (&x)[8]) {
+        if (i + 8 <= len) {
+            const f4u_t lo = *reinterpret_cast<const f4u_t*>(arow + i), hi = *reinterpret_cast<const f4u_t*>(arow + i + 4);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                x[c] = lo[c];
+                x[c + 4] = hi[c];
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < 8; ++c) x[c] = i + c < len ? arow[i + c] : 0.0f;
+        }
+    };
+    float amax = 0.0f;
+    for (int i = 8 * j; i < bs; i += 32) {
+        float x[8];
+        load8(i, x);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) amax = fmaxf(amax, fabsf(x[c]));
+    }
+    amax = fmaxf(amax, __shfl_xor(amax, 1, 4));
+    amax = fmaxf(amax, __shfl_xor(amax, 2, 4));
+    const float s = amax / 127.0f;
+    const float inv = s > 0.0f ? 1.0f / s : 0.0f;
+    const int t = m / (16 * nf), f = (m / 16) % nf, r = m & 15;
+    uint8_t* const tile = img + (int64_t)t * G * w4a8_image_bytes(nf);
+    for (int i = 8 * j; i < bs; i += 32) {
+        float x[8];
+        load8(i, x);
+        _Float16 q[8];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            int v = (int)__builtin_rintf(x[c] * inv);
+            v = max(-127, min(127, v));
+            q[c] = (_Float16)(float)(i + c < len ? v : 0);
+        }
+        const int step = (k0 + i) >> 5;
+        uint8_t* const image = tile + (int64_t)(step >> 2) * w4a8_image_bytes(nf);
+        *reinterpret_cast<half8_t*>(image + (((step & 3) * nf + f) * 64 + r + 16 * j) * 16) =
+            half8_t{q[0], q[4], q[1], q[5], q[2], q[6], q[3], q[7]};
+        if (j == 0)
+            *reinterpret_cast<float*>(image + 4096 * nf + (((step & 3) * 16 + r) * nf + f) * 4) = s;
+    }
+}
 
 struct W4a8MfmaParams {
     RawLayout L;
-    W4a8Args A;
+    const uint8_t* img;   // w4a8_stage_kernel's images [tiles_m][G]
     float* y;
-    int tiles_m, tiles_n;
+    int M, G, tiles_m, tiles_n;
 };
 
-__global__ __launch_bounds__(256) void mfma_w4a8_kernel(W4a8MfmaParams p)
+// x[b] of lane row s <-> x[s] of lane row b (rows of 16 lanes).
+__device__ __forceinline__ void transpose4(u32x4_t& x)
 {
-    constexpr int NF = kW8BN / 32;
-    const RawLayout& L = p.L;
-    __shared__ __attribute__((aligned(16))) uint32_t Bw[2][kW8BN][8];   // 32 signed codes per row
-    __shared__ float Sw[2][kW8BN];
-
-    const int tile = xcd_tile(blockIdx.x, p.tiles_m * p.tiles_n);
-    if (tile >= p.tiles_m * p.tiles_n) return;
-    const int m0 = (tile / p.tiles_n) * kW8BM, n0 = (tile % p.tiles_n) * kW8BN;
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-    const int spb = L.bs >> 5;
-    const int C = L.nb * spb;   // 32-code steps over padK
-    const int64_t row_bytes = (int64_t)L.nb * L.blob;
-
-    // producer: row pn of the tile, codes [8 ph, 8 ph + 8) of each step
-    const int pn = tid >> 2, ph = tid & 3;
-    const int prow = min(n0 + pn, L.N - 1);
-    const uint8_t* brow = L.b + (int64_t)prow * row_bytes + 4 * ph;
-    auto produce = [&](int bk, int s, int buf) {
-        const uint32_t x = *reinterpret_cast<const uint32_t*>(brow + (int64_t)bk * L.blob + 16 * s);
-        const uint32_t z4 = (uint32_t)w4a8_zp4(L, prow, bk) * 0x01010101u;
-        uint32_t ev, od;
-        w4a8_codes(x, z4, ev, od);
-        Bw[buf][pn][2 * ph] = ev;
-        Bw[buf][pn][2 * ph + 1] = od;
-        if (ph == 0) Sw[buf][pn] = L.scales[(int64_t)prow * L.nb + bk];
+    auto s32 = [&](int a, int b) {
+        const auto r = __builtin_amdgcn_permlane32_swap(x[a], x[b], false, false);
+        x[a] = r[0];
+        x[b] = r[1];
     };
+    auto s16 = [&](int a, int b) {
+        const auto r = __builtin_amdgcn_permlane16_swap(x[a], x[b], false, false);
+        x[a] = r[0];
+        x[b] = r[1];
+    };
+    s32(0, 2);
+    s32(1, 3);
+    s16(0, 1);
+    s16(2, 3);
+}
 
-    // consumer: lane -> A row (l % 32), 16-byte k slot (l / 32) of each step
-    const int am = min(m0 + wave * 32 + (lane & 31), p.A.M - 1);
-    const int8_t* pa = p.A.aq + (int64_t)am * p.A.padK + 16 * (lane >> 5);
-    // rows of the lane's 16 outputs: rbase + 8 (v / 4) + v % 4; groups of 4 rows read as one
-    // float4 of the transposed activation scales (clamped into the array past M)
-    const int rbase = m0 + wave * 32 + 4 * (lane >> 5);
-    int sa_off[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) sa_off[q] = min(rbase + 8 * q, p.A.Mp - 4);
+// SPB: steps per block, 1 or 2, 4 for any multiple of 4, 0 for any number.
+template <int NF, int SPB>
+__global__ __launch_bounds__(256, 2) void mfma_w4a8_kernel(W4a8MfmaParams p)
+{
+    constexpr int IMG = w4a8_image_bytes(NF);
+    extern __shared__ __attribute__((aligned(16))) uint8_t w4a8_lds[];
+    const RawLayout& L = p.L;
+    const int tile = xcd_tile(blockIdx.x, p.tiles_m * p.tiles_n);   // an XCD's range shares weight rows
+    if (tile >= p.tiles_m * p.tiles_n) return;
+    const int mt = tile % p.tiles_m, nt = tile / p.tiles_m;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int ln = lane & 15, ls = lane >> 4;
+    const int n0 = nt * kW8BN + 16 * wave;
+    const int live = __builtin_amdgcn_readfirstlane(max(0, min(16, L.N - n0)));   // this wave's weight rows (in an SGPR)
+    const int spb = L.bs >> 5, C = L.nb * spb;
+    const int row_bytes = L.nb * L.blob;
 
-    float facc[NF][16];
-#pragma unroll
-    for (int j = 0; j < NF; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) facc[j][v] = 0.0f;
-    v16i_t iacc[NF];
-#pragma unroll
-    for (int j = 0; j < NF; ++j) iacc[j] = v16i_t{};
+    // resources over this wave's rows alone: loads past them (and steps past the last row) read zero
+    const int nr = __builtin_amdgcn_readfirstlane(min(n0, L.N - 1));
+    const __amdgpu_buffer_rsrc_t rb = buffer_rsrc(L.b + (int64_t)nr * row_bytes, live * row_bytes);
+    const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(L.scales + (int64_t)nr * L.nb, live * L.nb * 4);
+    const __amdgpu_buffer_rsrc_t rz = buffer_rsrc(L.zp ? L.zp + (int64_t)nr * L.zrb : L.b, L.zp ? live * L.zrb : 0);
+    const __amdgpu_buffer_rsrc_t ra = buffer_rsrc(p.img + (int64_t)mt * p.G * IMG, p.G * IMG);
+    const uint32_t lds0 = lds_address(w4a8_lds);
+    auto load_a = [&](int g) {
+        for (int i = wave; i < IMG / 1024; i += 4)
+            lds_load16(ra, 16 * lane, g * IMG + 1024 * i, lds0 + (g & 1) * IMG + 1024 * i);
+    };
+    static_assert(IMG % 1024 == 0, "images are copied in whole KB");
 
-    v4i_t a_next = *reinterpret_cast<const v4i_t*>(pa);
-    produce(0, 0, 0);
-    __syncthreads();
-    int t = 0;   // 32-code step; buffer t & 1
-    for (int bk = 0; bk < L.nb; ++bk) {
-        float4 sa4[4];   // the block's activation scales, read while its steps run
+    // group g's codes (step 4 g + ls of row ln) and, for the blocks its steps lie in, scales of
+    // rows 4 ls + v and zero points of row ln
+    constexpr int NB = SPB == 2 ? 2 : SPB == 4 ? 1 : 4;
+    struct Group {
+        u32x4_t x;
+        float sw[NB][4];
+        uint32_t z[NB];
+    };
+    auto load_w = [&](int g, Group& w) {
+        w.x = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rb, ln * row_bytes + 64 * g + 16 * ls, 0, 0));
+        if constexpr (SPB == 1 || SPB == 2) {   // neighbouring blocks
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            sa4[q] = *reinterpret_cast<const float4*>(p.A.sat + (int64_t)bk * p.A.Mp + sa_off[q]);
-        for (int s = 0; s < spb; ++s, ++t) {
-            const int buf = t & 1;
-            const v4i_t a_cur = a_next;
-            if (t + 1 < C) a_next = *reinterpret_cast<const v4i_t*>(pa + 32 * (t + 1));
+            for (int v = 0; v < 4; ++v) {
+                const int off = ((4 * ls + v) * L.nb + NB * g) * 4;
+                if constexpr (SPB == 1) {
+                    const auto s4 = __builtin_bit_cast(floatx4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
 #pragma unroll
-            for (int j = 0; j < NF; ++j) {
-                const v4i_t b = *reinterpret_cast<const v4i_t*>(&Bw[buf][32 * j + (lane & 31)][4 * (lane >> 5)]);
-                iacc[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a_cur, b, iacc[j], 0, 0, 0);
-            }
-            if (s == spb - 1) {   // the block's end: its terms join the fp32 sums, in block order
-#pragma unroll
-                for (int j = 0; j < NF; ++j) {
-                    const float sw = Sw[buf][32 * j + (lane & 31)];
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const float sq[4] = {sa4[q].x, sa4[q].y, sa4[q].z, sa4[q].w};
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const int v = 4 * q + i;
-                            const float pr = sq[i] * sw;
-                            facc[j][v] = facc[j][v] + pr * (float)iacc[j][v];
-                        }
-                    }
-                    iacc[j] = v16i_t{};
+                    for (int b = 0; b < 4; ++b) w.sw[b][v] = s4[b];
+                } else {
+                    w.sw[0][v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0));
+                    w.sw[NB - 1][v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, off + 4, 0, 0));
                 }
             }
-            if (t + 1 < C) {
-                if (s + 1 < spb) produce(bk, s + 1, buf ^ 1);
-                else produce(bk + 1, 0, buf ^ 1);
+#pragma unroll
+            for (int h = 0; h < NB / 2; ++h) {
+                const uint32_t z = __builtin_amdgcn_raw_buffer_load_b8(rz, ln * L.zrb + NB / 2 * g + h, 0, 0);
+                w.z[2 * h] = z & 15;
+                w.z[2 * h + 1] = z >> 4;
             }
-            __syncthreads();
+        } else {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const int bk = (4 * g + b) / spb;
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    w.sw[b][v] = __builtin_bit_cast(
+                        float, __builtin_amdgcn_raw_buffer_load_b32(rs, ((4 * ls + v) * L.nb + bk) * 4, 0, 0));
+                w.z[b] = (__builtin_amdgcn_raw_buffer_load_b8(rz, ln * L.zrb + (bk >> 1), 0, 0) >> (4 * (bk & 1))) & 15;
+            }
         }
-    }
+    };
 
+    floatx4_t acc[NF], dot[NF];
 #pragma unroll
-    for (int j = 0; j < NF; ++j) {
-        const int col = n0 + 32 * j + (lane & 31);
-        if (col < L.N) {
+    for (int f = 0; f < NF; ++f) acc[f] = dot[f] = floatx4_t{};
+    int in_block = 0;   // steps of the current block done
+
+    Group w;
+    load_a(0);
+    load_w(0, w);
+    for (int g = 0; g < p.G; ++g) {
+        wait_vmcnt<0>();   // this wave's part of the image, and its weights
+        lds_barrier();     // everyone's; and the readers of the other image are done
+        Group nx = w;
+        if (g + 1 < p.G) {
+            load_a(g + 1);
+            load_w(g + 1, nx);
+        }
+        const uint8_t* const lds = w4a8_lds + (g & 1) * IMG;
+        transpose4(w.x);
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int row = rbase + 8 * (v >> 2) + (v & 3);
-                if (row < p.A.M) p.y[(int64_t)row * L.N + col] = facc[j][v];
+        for (int b = 0; b < 4; ++b) {
+            if (4 * g + b >= C) break;   // the last group's padding
+            const int k = b * NB / 4;   // the step's block
+            const uint32_t zp = L.zp ? w.z[k] : 8u;
+            const h2_t zb = zp_half2(zp);
+            uint32_t d[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) d[t] = as_u32(as_h2(and_or(w.x[b] >> (4 * t), 0x000F000Fu, kHalfMagic)) - zb);
+            const half8_t wv = __builtin_bit_cast(half8_t, u32x4_t{d[0], d[1], d[2], d[3]});
+            const uint8_t* const la = lds + (b * NF * 64 + lane) * 16;
+#pragma unroll
+            for (int f = 0; f < NF; ++f) {
+                const half8_t av = *reinterpret_cast<const half8_t*>(la + f * 1024);
+                dot[f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv, av, SPB == 1 ? floatx4_t{} : dot[f], 0, 0, 0);
             }
+            if (SPB == 1 || (SPB == 2 && (b & 1)) || ((SPB == 0 || (SPB == 4 && b == 3)) && (in_block += SPB ? SPB : 1) == spb)) {
+                // the block's terms join the fp32 sums, in block order
+                const float* const sa = reinterpret_cast<const float*>(lds + 4096 * NF) + (b * 16 + ln) * NF;
+#pragma unroll
+                for (int f = 0; f < NF; ++f) {
+                    const float s = sa[f];
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const float pr = s * w.sw[k][v];
+                        acc[f][v] = acc[f][v] + pr * dot[f][v];
+                    }
+                    if (SPB != 1) dot[f] = floatx4_t{};
+                }
+                in_block = 0;
+            }
+        }
+        w = nx;
+    }
+    // acc[f][v] is Y[16 f + ln][n0 + 4 ls + v]
+    typedef float f4u_t __attribute__((ext_vector_type(4), aligned(4)));
+    const int n = n0 + 4 * ls;
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+        const int m = mt * 16 * NF + 16 * f + ln;
+        if (m >= p.M) continue;
+        float* const o = p.y + (int64_t)m * L.N + n;
+        if (n + 4 <= L.N) {
+            *reinterpret_cast<f4u_t*>(o) = f4u_t{acc[f][0], acc[f][1], acc[f][2], acc[f][3]};
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (n + v < L.N) o[v] = acc[f][v];
         }
     }
 }

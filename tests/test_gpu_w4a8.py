@@ -189,3 +189,18 @@ def test_w4a8_within_the_bar_of_the_managed_variant(gpu, op, M):
     log(f"  rel-L2 {rel:.3e} cosine {cos:.9f}")
     assert rel < 0.03 and cos > 0.999, (rel, cos)
     assert rel < 1e-3, rel
+
+
+# mfma_w4a8: every block length its launches tell apart (1, 2, 3, 4 and 8 steps of 32 codes)
+# at launches wide enough for its taller tiles (32, 64 and 128 rows), with a last group of
+# steps, last rows and last columns that are not full.
+@pytest.mark.parametrize("bs", [32, 64, 96, 128, 256])
+@pytest.mark.parametrize("M,N", [(65, 16406), (129, 8450), (300, 5000)])
+def test_w4a8_tiles_bit_exact(gpu, bs, M, N):
+    op = Op("tiles", 808, N, bs, bs != 128)
+    b, s, z = workloads.make_weights(op, seed=bs + M)
+    a = workloads.make_activations(M, op.K, seed=M, kind="rmsnorm")
+    w = native.NBitsWeights(b, s, z, op.N, op.K, op.bits, op.block_size)
+    log(f"w4a8 bs={bs} M={M} N={N} {w.launch_info_w4a8(M)}")
+    assert np.array_equal(w.gemm_w4a8(a), oracle.qgemm_w4a8(a, b, s, z, op.N, op.K, op.bits, op.block_size))
+    w.close()
