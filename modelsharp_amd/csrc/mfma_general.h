@@ -1,6 +1,8 @@
 // mfma_general.h — GEMM (M > 16) on the matrix cores for the weight formats the 4-bit
 // kernels do not take: bits = 8, float zero points, block sizes other than 32/64/128/256,
-// K not a multiple of 32 (K and the block size multiples of 8). At fp32-level accuracy:
+// K not a multiple of 32 (K and the block size multiples of 8).
+// Block sizes 16, 32, ..., 512 go to mfma_block.h when the call has a workspace; the others,
+// and calls without one, come here. At fp32-level accuracy:
 //   * the producer dequantizes every weight exactly as the reference does
 //     (W = fl(fl(q - zp) * s), generic_nbits.h) and splits it into fp16 halves,
 //     W = 2^f[n] (Wh + Wl), with the row exponent f[n] (precomputed per weights handle)

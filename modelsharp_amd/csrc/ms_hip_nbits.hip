@@ -15,7 +15,9 @@
 //   other formats (bits 8, float zero points, other block sizes or K), K and the block
 //   size multiples of 8:
 //     M <= 16                                                 -> gemv_general
-//     M >  16                                                 -> mfma_general (exact)
+//     M >  16                                                 -> mfma_general (exact): with a
+//                                                                workspace and block sizes 16,
+//                                                                32, ..., 512 mfma_block's kernel
 //   anything else                                             -> generic
 // Declarations and reference citations: include/ms_hip_kernels.h.
 #include "../../include/ms_hip_kernels.h"
@@ -48,6 +50,7 @@
 #include "gemv_w4.h"
 #include "gemv_w4_panel.h"
 #include "generic_nbits.h"
+#include "mfma_block.h"
 #include "mfma_general.h"
 #include "w4a8.h"
 #include "gqa_split.h"
@@ -233,6 +236,16 @@ struct Weights {
     uint8_t* d_zp = nullptr;
     float* d_zpf = nullptr;     // float zero points [N * nb]
     int* d_wexp = nullptr;      // general formats: row exponents of the weights [N]
+    // mfma_block's workspaces, one per stream that has called (the format's calls may overlap on
+    // several streams: mfma_general, which further streams and captured calls get, needs none)
+    struct BlockSlot {
+        hipStream_t stream = nullptr;
+        uint8_t* data = nullptr;
+        size_t bytes = 0;
+    };
+    std::mutex block_mu;
+    std::array<BlockSlot, 4> block_slots;
+    int block_used = 0;
     // mfma_w4_rb's chunk-major scales / zero points [K / 128][N][4], built by the first
     // eager call that takes it (rb_ready then 1; guarded by ws_mu)
     uint32_t* d_sz4 = nullptr;
@@ -325,6 +338,11 @@ void free_weights(Weights& w)
     if (w.d_zp) (void)hipFree(w.d_zp);
     if (w.d_zpf) (void)hipFree(w.d_zpf);
     if (w.d_wexp) (void)hipFree(w.d_wexp);
+    for (auto& b : w.block_slots) {
+        if (b.data) (void)hipFree(b.data);
+        b.data = nullptr;
+        b.bytes = 0;
+    }
     if (w.d_stage) (void)hipFree(w.d_stage);
     if (w.h_stage) (void)hipHostFree(w.h_stage);
     if (w.h_err) (void)hipHostFree(w.h_err);
@@ -1481,6 +1499,118 @@ int ensure_rb_layout(Weights& w, hipStream_t stream)
     return 1;
 }
 
+// ---- mfma_block: the general formats with block sizes 16, 32, ..., 512 -----------------------
+// Needs a workspace (A's images); where none can be had mfma_general takes the call.
+bool block_eligible(const Weights& w)
+{
+    const int64_t G = ((int64_t)w.nb * w.bs + 63) / 64;
+    return general_eligible(w) && w.bs >= 16 && w.bs <= 512 && (w.bs & (w.bs - 1)) == 0 &&
+           64 * (int64_t)w.nb * w.blob < kPipeFar && 64 * (int64_t)w.nb * 4 < kPipeFar &&
+           2 * G * kBlkImage < kPipeFar;
+}
+
+// Tiles of 64 x 128 from two per CU on (a lone wave on a SIMD issues a VALU instruction in 6 to 7
+// cycles, two of them one in 4), else 32 x 64 with K over the four waves.
+bool block_whole_k(const Weights& w, int M)
+{
+    return (int64_t)((M + 63) / 64) * ((w.N + 127) / 128) >= 2 * device_cus();
+}
+
+struct BlockWs {
+    int G = 0;
+    size_t rexp_off = 0, total = 0;
+};
+
+BlockWs block_ws(const Weights& w, int M)
+{
+    BlockWs L;
+    L.G = (int)(((int64_t)w.nb * w.bs + 63) / 64);
+    L.rexp_off = (size_t)((M + 31) / 32) * L.G * kBlkImage;
+    L.total = L.rexp_off + align256((size_t)M * sizeof(int));
+    return L;
+}
+
+typedef void (*BlockFn)(BlockParams);
+template <bool B8, bool FZ, int BL>
+BlockFn block_fn(bool whole_k)
+{
+    return whole_k ? mfma_block_kernel<B8, FZ, BL, 2, 2, 1> : mfma_block_kernel<B8, FZ, BL, 1, 1, 4>;
+}
+template <bool B8, bool FZ>
+BlockFn block_fn(int bs, bool whole_k)
+{
+    return bs == 16 ? block_fn<B8, FZ, 4>(whole_k) : bs == 32 ? block_fn<B8, FZ, 5>(whole_k)
+           : bs == 64 ? block_fn<B8, FZ, 6>(whole_k) : block_fn<B8, FZ, 7>(whole_k);
+}
+
+// The stream's workspace of at least `bytes`, under block_mu; nullptr while the stream is being
+// captured (a graph may be replayed beside other calls), for the per-thread stream (one value
+// that names many streams), for a fifth stream, and when memory is short.
+uint8_t* block_workspace(Weights& w, size_t bytes, hipStream_t stream)
+{
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (stream == hipStreamPerThread || hipStreamIsCapturing(stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    int i = 0;
+    while (i < w.block_used && w.block_slots[i].stream != stream) ++i;
+    if (i == (int)w.block_slots.size()) return nullptr;
+    auto& b = w.block_slots[i];
+    if (b.bytes < bytes) {
+        // earlier launches on this stream may still use the old buffer
+        if (b.data && (hipStreamSynchronize(stream) != hipSuccess || hipFree(b.data) != hipSuccess)) return nullptr;
+        b.data = nullptr;
+        b.bytes = 0;
+        if (hipMalloc(&b.data, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            b.data = nullptr;
+            return nullptr;
+        }
+        b.bytes = bytes;
+    }
+    if (i == w.block_used) {
+        b.stream = stream;
+        ++w.block_used;
+    }
+    return b.data;
+}
+
+// Returns 1 when the call is not taken (mfma_general is to take it).
+int launch_mfma_block(Weights& w, const float* dA, float* dY, int M, hipStream_t stream)
+{
+    if (!block_eligible(w)) return 1;
+    const BlockWs B = block_ws(w, M);
+    std::lock_guard<std::mutex> lock(w.block_mu);   // held over both launches: they share the workspace
+    uint8_t* const data = block_workspace(w, B.total, stream);
+    if (!data) return 1;
+    const bool whole = block_whole_k(w, M);
+    BlockParams p;
+    p.L = raw_layout(w);
+    p.wexp = w.d_wexp;
+    p.img = data;
+    p.rexp = reinterpret_cast<const int*>(data + B.rexp_off);
+    p.y = dY;
+    p.M = M;
+    p.G = B.G;
+    p.log2bs = log2_exact(w.bs);
+    p.tiles_m = (M + (whole ? 63 : 31)) / (whole ? 64 : 32);
+    p.tiles_n = (w.N + (whole ? 127 : 63)) / (whole ? 128 : 64);
+    const unsigned rows = (unsigned)((M + 32 * kXcds - 1) / (32 * kXcds) * (32 * kXcds));
+    hipLaunchKernelGGL(block_stage_a_kernel, dim3(rows), dim3(256), 0, stream, dA, data,
+                       reinterpret_cast<int*>(data + B.rexp_off), M, w.K, B.G, p.log2bs);
+    MS_HIP_CHECK(hipGetLastError());
+    const bool fz = w.zp_float;
+    const BlockFn fn = w.bits == 8 ? (fz ? block_fn<true, true>(w.bs, whole) : block_fn<true, false>(w.bs, whole))
+                                   : (fz ? block_fn<false, true>(w.bs, whole) : block_fn<false, false>(w.bs, whole));
+    const int lds = (whole ? 4 : 8) * kBlkImage, tiles = p.tiles_m * p.tiles_n;
+    if (lds > 64 * 1024)
+        MS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    hipLaunchKernelGGL(fn, dim3(((tiles + kXcds - 1) / kXcds) * kXcds), dim3(256), lds, stream, p);
+    MS_HIP_CHECK(hipGetLastError());
+    return MS_HIP_OK;
+}
+
 // ---- dispatch ------------------------------------------------------------------------------
 // Which kernel a call with M rows takes (ids of ms_hip_nbits_launch_info).
 enum KernelId {
@@ -1537,12 +1667,17 @@ KernelId workspace_free_kernel(const Weights& w, const Knobs& kn, int M)
 }
 
 int launch_kernel(Weights& w, const Knobs& kn, KernelId k, const Ws& ws, const float* dA, float* dY, int M,
-                  hipStream_t stream, AConv* conv = nullptr)
+                  hipStream_t stream, AConv* conv = nullptr, bool may_alloc = true)
 {
     switch (k) {
         case kGeneric: return launch_generic(w, dA, dY, M, stream);
         case kGemvGeneral: return launch_gemv_general(w, dA, dY, M, stream);
-        case kMfmaGeneral: return launch_mfma_general(w, dA, dY, M, stream);
+        case kMfmaGeneral:
+            if (may_alloc) {
+                const int r = launch_mfma_block(w, dA, dY, M, stream);
+                if (r != 1) return r;
+            }
+            return launch_mfma_general(w, dA, dY, M, stream);
         case kGemvW8: return launch_gemv_w8(w, kn, dA, dY, M, stream);
         case kGemv:
         case kPanel: return launch_gemv(w, kn, dA, dY, M, stream);
@@ -2217,7 +2352,7 @@ int ms_hip_nbits_gemm_dev_noalloc(void* handle, const float* dA, float* dY, int 
         // at zero (a fill kernel, which a captured graph can hold).
         if ((st = zero_ints(ws.cnt, (int64_t)need_c, s))) return st;
     }
-    return launch_kernel(*w, kn, k, ws, dA, dY, M, s);
+    return launch_kernel(*w, kn, k, ws, dA, dY, M, s, nullptr, false);
 }
 
 int ms_hip_nbits_device_error(void* handle)
@@ -2839,6 +2974,8 @@ int ms_hip_nbits_launch_info(void* handle, int M, int* kernel_id, int* lanes_per
         }
         case kMfmaGeneral:
             gr = ((M + kGenBM - 1) / kGenBM) * ((w->N + kGenBN - 1) / kGenBN);
+            if (block_eligible(*w))
+                gr = block_whole_k(*w, M) ? ((M + 63) / 64) * ((w->N + 127) / 128) : ((M + 31) / 32) * ((w->N + 63) / 64);
             gr = ((gr + kXcds - 1) / kXcds) * kXcds;
             break;
         case kSkinny: gr = ((w->N + kSkinnyRows - 1) / kSkinnyRows) * skinny_ksw(*w, kn); break;

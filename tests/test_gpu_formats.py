@@ -541,3 +541,32 @@ def test_skinny_8bit(gpu, zp, K, ksw, bs):
         w.set_tuning(4, 0)
         w.set_tuning(5, 0)
     w.close()
+
+
+# mfma_block (the general formats with block sizes 16 to 512): block ends inside and across
+# its 64-k groups, a last group and a last block that are not full, rows and columns past its
+# tiles, and both launch shapes (64 x 128 tiles from one tile per CU on, else 32 x 64 with K
+# over four waves).
+BLOCK_OPS = [
+    Op("b4_bs16_k24", 24, 70, 16, True),
+    Op("b4_bs256", 1032, 129, 256, True),
+    Op("b8_bs16_sym", 200, 65, 16, False, bits=8),
+    Op("b4_bs16_wide", 72, 16500, 16, True),
+    Op("b4_bs512", 1544, 64, 512, False),
+    Op("b4_bs64_wide", 200, 16402, 64, True),
+    Op("b8_bs32_wide", 104, 16390, 32, True, bits=8),
+]
+
+
+@pytest.mark.parametrize("fzp", [False, True], ids=["zp", "float_zp"])
+@pytest.mark.parametrize("op", BLOCK_OPS, ids=lambda o: o.name)
+@pytest.mark.parametrize("M", [17, 64, 97])
+def test_block_gemm(gpu, op, M, fzp):
+    b, s, z = workloads.make_weights(op, seed=op.K + M)
+    zpf = float_zero_points(op, seed=op.N + M) if fzp else None
+    z = None if fzp else z
+    a = workloads.make_activations(M, op.K, seed=M + 3, kind="rmsnorm")
+    w = native.NBitsWeights(b, s, zpf if fzp else z, op.N, op.K, op.bits, op.block_size)
+    log(f"block {op.name} M={M} {w.launch_info(M)}")
+    check_against_oracle(w, a, b, s, z, zpf, op, f"{op.name} M={M}")
+    w.close()
