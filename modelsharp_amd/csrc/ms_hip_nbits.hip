@@ -917,8 +917,37 @@ constexpr std::array<GenGemvFn, sizeof...(I)> gen_gemv_table(std::index_sequence
 }
 constexpr auto kGenGemvTable = gen_gemv_table(std::make_index_sequence<16>{});
 
+template <bool B8, size_t... I>
+constexpr std::array<void (*)(RawLayout, const float*, float*, int, int), sizeof...(I)> gen_chunk_table(
+    std::index_sequence<I...>)
+{
+    return {gemv_chunk_kernel<(int)I + 1, B8>...};
+}
+constexpr auto kGenChunk4Table = gen_chunk_table<false>(std::make_index_sequence<16>{});
+constexpr auto kGenChunk8Table = gen_chunk_table<true>(std::make_index_sequence<16>{});
+
+int log2_exact(int v);
+
+// gemv_chunk_kernel: blocks of whole 16-byte chunks of codes, a power of two of them (so that
+// every chunk lies in one block and is 16-byte aligned).
+bool gemv_chunk_fits(const Weights& w)
+{
+    const int chunk = w.bits == 8 ? 16 : 32;
+    return w.bs % chunk == 0 && log2_exact(w.bs / chunk) >= 0;
+}
+
 int launch_gemv_general(const Weights& w, const float* dA, float* dY, int M, hipStream_t stream)
 {
+    if (gemv_chunk_fits(w)) {
+        const int chunk = w.bits == 8 ? 16 : 32, C = (w.K + chunk - 1) / chunk;
+        const int tile = std::min(C, kGenPanelBytes / (M * chunk * (int)sizeof(float)));
+        const auto fn = (w.bits == 8 ? kGenChunk8Table : kGenChunk4Table)[M - 1];
+        hipLaunchKernelGGL(fn, dim3((w.N + kGenChunkRows - 1) / kGenChunkRows), dim3(512),
+                           (size_t)M * tile * chunk * sizeof(float), stream, raw_layout(w), dA, dY,
+                           log2_exact(w.bs / chunk), tile);
+        MS_HIP_CHECK(hipGetLastError());
+        return MS_HIP_OK;
+    }
     hipLaunchKernelGGL(kGenGemvTable[M - 1], dim3((w.N + kGenRowsPerWg - 1) / kGenRowsPerWg), dim3(256), 0, stream,
                        raw_layout(w), dA, dY);
     MS_HIP_CHECK(hipGetLastError());
@@ -1576,14 +1605,14 @@ uint8_t* block_workspace(Weights& w, size_t bytes, hipStream_t stream)
     return b.data;
 }
 
-// Returns 1 when the call is not taken (mfma_general is to take it).
+// Returns -1 when the call is not taken (mfma_general is to take it).
 int launch_mfma_block(Weights& w, const float* dA, float* dY, int M, hipStream_t stream)
 {
-    if (!block_eligible(w)) return 1;
+    if (!block_eligible(w)) return -1;
     const BlockWs B = block_ws(w, M);
     std::lock_guard<std::mutex> lock(w.block_mu);   // held over both launches: they share the workspace
     uint8_t* const data = block_workspace(w, B.total, stream);
-    if (!data) return 1;
+    if (!data) return -1;
     const bool whole = block_whole_k(w, M);
     BlockParams p;
     p.L = raw_layout(w);
@@ -1675,7 +1704,7 @@ int launch_kernel(Weights& w, const Knobs& kn, KernelId k, const Ws& ws, const f
         case kMfmaGeneral:
             if (may_alloc) {
                 const int r = launch_mfma_block(w, dA, dY, M, stream);
-                if (r != 1) return r;
+                if (r >= 0) return r;
             }
             return launch_mfma_general(w, dA, dY, M, stream);
         case kGemvW8: return launch_gemv_w8(w, kn, dA, dY, M, stream);
@@ -2964,7 +2993,13 @@ int ms_hip_nbits_launch_info(void* handle, int M, int* kernel_id, int* lanes_per
     int G = 0, gr = 0, bl = 256;
     switch (kid) {
         case kGeneric: gr = (int)(((int64_t)M * w->N + 255) / 256); break;
-        case kGemvGeneral: gr = (w->N + kGenRowsPerWg - 1) / kGenRowsPerWg; G = 16; break;
+        case kGemvGeneral: {
+            const int rows = gemv_chunk_fits(*w) ? kGenChunkRows : kGenRowsPerWg;
+            gr = (w->N + rows - 1) / rows;
+            G = 16;
+            if (gemv_chunk_fits(*w)) bl = 512;
+            break;
+        }
         case kGemvW8: {
             const int ci = pick_gemv8_config(*w, kn, M);
             G = kGemv8Configs[ci].G;

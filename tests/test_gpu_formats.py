@@ -570,3 +570,18 @@ def test_block_gemm(gpu, op, M, fzp):
     log(f"block {op.name} M={M} {w.launch_info(M)}")
     check_against_oracle(w, a, b, s, z, zpf, op, f"{op.name} M={M}")
     w.close()
+
+
+# gemv_chunk_kernel: rows of one chunk, of whole batches (16 lanes x 4 chunks) and one more, and
+# panels of more than one tile of K; rows past its 32 per workgroup.
+@pytest.mark.parametrize("bits,K", [(4, 24), (4, 2048), (4, 2088), (8, 16), (8, 1024), (8, 1048)])
+@pytest.mark.parametrize("M", [1, 5, 16])
+def test_chunk_gemv(gpu, M, bits, K):
+    op = Op("chunk", K, 37, 32, True, bits=bits)
+    b, s, _ = workloads.make_weights(op, seed=K + M)
+    zpf = float_zero_points(op, seed=K)
+    a = workloads.make_activations(M, K, seed=M)
+    w = native.NBitsWeights(b, s, zpf, op.N, op.K, op.bits, op.block_size)
+    kernel, _ = check_against_oracle(w, a, b, s, None, zpf, op, f"chunk bits={bits} K={K} M={M}")
+    assert kernel == "gemv_general"
+    w.close()
