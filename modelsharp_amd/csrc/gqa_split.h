@@ -31,7 +31,7 @@
 // 28 / 4 heads of 128, 2048 queries and keys: 126 us with the conversion (14 us of it),
 // 239 TFLOP/s of causal work, where gqa_flash_kernel took 637; its error against 64 bits is
 // 2.7e-7 (4.5e-7). 32 / 8 heads of 96 over 1000 tokens: 60 us, 1111 before
-// (gqa_attention_kernel). The MFMAs are busy 31% of the time, the VALU (680 instructions per
+// (gqa_attention_kernel). The MFMAs are busy 31% of the time, the VALU (630 instructions per
 // wave and chunk) as much: what is left is the waits at each phase's barrier.
 // What the halves cannot carry (an infinity, a NaN, |q| or |k| >= 2^50, key or value rows
 // more than 2^12 apart in one scale: a row seen by queries that do not see the larger one
