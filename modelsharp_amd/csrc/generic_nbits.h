@@ -10,17 +10,10 @@
 // (len = min(bs, K - b*bs), :246). W = ((float)q - zp) * scale, each operation rounded
 // in fp32 (MatMulNBitsSimd.cs:100-111): bit for bit the reference's weights.
 #pragma once
+#include "formats.h"
 #include "nbits_device.h"
 
 namespace msnb {
-
-struct RawLayout {
-    const uint8_t* b;
-    const float* scales;
-    const uint8_t* zp;   // packed codes, or nullptr
-    const float* zpf;    // float zero points [N * nb], or nullptr (then zp, else 2^(bits-1))
-    int N, K, bits, bs, nb, blob, zrb;
-};
 
 __device__ __forceinline__ int unpack_code(const uint8_t* data, int64_t base, int index, int bits)
 {

@@ -38,8 +38,8 @@
 // would lose its low bits) sends the query blocks that meet it to gqa_split_plain(), plain
 // fp32 arithmetic row by row.
 #pragma once
-#include "gqa.h"
-#include "mfma_w4_pipe.h"
+#include "gqa_args.h"
+#include "mfma_device.h"
 
 namespace msnb {
 

@@ -28,7 +28,7 @@
 //                         barrier per 64 k.
 #pragma once
 #include "generic_nbits.h"
-#include "mfma_w4_pipe.h"
+#include "mfma_device.h"
 
 namespace msnb {
 

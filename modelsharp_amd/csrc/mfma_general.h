@@ -20,7 +20,7 @@
 // memory in the MFMA operand layout, one step ahead, and splits them in registers.
 #pragma once
 #include "generic_nbits.h"
-#include "mfma_w4.h"
+#include "mfma_device.h"
 
 namespace msnb {
 

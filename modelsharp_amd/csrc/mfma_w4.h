@@ -33,12 +33,9 @@
 #pragma once
 #include <cmath>
 
-#include "nbits_device.h"
+#include "mfma_device.h"
 
 namespace msnb {
-
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef float floatx16_t __attribute__((ext_vector_type(16)));
 
 struct MfmaParams {
     const uint8_t* b;
@@ -55,17 +52,6 @@ struct MfmaParams {
 };
 
 constexpr int kMfmaThreads = 256;
-constexpr int kBsStride = 40;   // fp16 per LDS weight row (32 + 8 pad)
-constexpr int kXcds = 8;
-
-// tile index of workgroup `bid` among tiles_m*tiles_n tiles (m-major), so that
-// XCD x = bid % 8 owns the contiguous tile range [x*per, (x+1)*per).
-__device__ __forceinline__ int xcd_tile(int bid, int tiles)
-{
-    const int per = (tiles + kXcds - 1) / kXcds;
-    return (bid % kXcds) * per + bid / kXcds;
-}
-
 // hi / lo halves of 8 activations times 2^-e, in the order k0,k4,k1,k5,k2,k6,k3,k7.
 __device__ __forceinline__ void split8(const float4& x03, const float4& x47, int e, half8_t& hi, half8_t& lo)
 {

@@ -95,40 +95,9 @@ struct PipeLds {
     static constexpr int BYTES = OFF_E + kPipeBM * 4;
     static_assert(BYTES <= 160 * 1024, "the pipelined prefill's LDS exceeds a CU's");
 };
-// Base offset of a row beyond the matrix: above every buffer the kernel reads
-// (the host checks each is smaller), so loads from it return zero.
-constexpr int kPipeFar = 0x40000000;
-
 __device__ __forceinline__ uint32_t pack_h2(float lo, float hi)
 {
     return __builtin_bit_cast(uint32_t, h2_t{(_Float16)lo, (_Float16)hi});
-}
-
-__device__ __forceinline__ float max_abs8(const float4& lo, const float4& hi)
-{
-    return fmaxf(fmaxf(fmaxf(fabsf(lo.x), fabsf(lo.y)), fmaxf(fabsf(lo.z), fabsf(lo.w))),
-                 fmaxf(fmaxf(fabsf(hi.x), fabsf(hi.y)), fmaxf(fabsf(hi.z), fabsf(hi.w))));
-}
-
-// Exponent e of a row whose largest magnitude is mx: mx * 2^-e lies in [2^14, 2^15)
-// (mx in [2^(E-1), 2^E) with E = frexp exponent, e = E - 15). Rows that are all zero,
-// or hold an inf (fmaxf skips NaN), take e = 0: their sums are zero or non-finite
-// whatever the scaling.
-__device__ __forceinline__ int row_exponent(float mx)
-{
-    return (mx > 0.0f && mx <= 3.402823466e38f) ? __builtin_amdgcn_frexp_expf(mx) - 15 : 0;
-}
-
-// Largest value of x over the workgroup of 256 threads, in every thread.
-__device__ __forceinline__ float block256_max(float x, float* red4)
-{
-    x = row16_max_all(x);
-    x = fmaxf(x, xor16_value(x));
-    x = fmaxf(x, xor32_value(x));
-    const int wave = threadIdx.x / kWave;
-    if ((threadIdx.x & (kWave - 1)) == 0) red4[wave] = x;
-    __syncthreads();
-    return fmaxf(fmaxf(red4[0], red4[1]), fmaxf(red4[2], red4[3]));
 }
 
 __device__ __forceinline__ u32x4_t pack_group(const float4& lo, const float4& hi, int e)
@@ -223,29 +192,6 @@ __device__ __forceinline__ void dequant8_f16_b8(uint32_t d0, uint32_t d1, h2_t z
         o[t] = as_u32((as_h2(and_or(pr, 0x00FF00FFu, kHalfMagic)) - zb) * s2);
     }
 }
-
-typedef __attribute__((address_space(3))) uint8_t lds_byte_t;
-__device__ __forceinline__ uint32_t lds_address(const void* p) { return (uint32_t)(uintptr_t)(lds_byte_t*)p; }
-
-// buffer -> LDS loads: lane i's bytes land at LDS m0 + 16*i (x4) or m0 + 4*i (ushort).
-__device__ __forceinline__ void lds_load16(__amdgpu_buffer_rsrc_t r, int voff, int soff, uint32_t m0v)
-{
-    asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff), "{m0}"(m0v) : "memory");
-}
-__device__ __forceinline__ void lds_load4(__amdgpu_buffer_rsrc_t r, int voff, int soff, uint32_t m0v)
-{
-    asm volatile("buffer_load_dword %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff), "{m0}"(m0v) : "memory");
-}
-__device__ __forceinline__ void lds_load2(__amdgpu_buffer_rsrc_t r, int voff, int soff, uint32_t m0v)
-{
-    asm volatile("buffer_load_ushort %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff), "{m0}"(m0v) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_vmcnt()
-{
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // 16-byte chunk slot of k-chunk j in row r: conflict-free for 8- and 16-row passes.
 __device__ __forceinline__ int pipe_slot(int r, int j) { return j ^ (((r >> 2) & 3) ^ (r & 2)); }

@@ -45,15 +45,10 @@
 #include <strings.h>
 #include <unistd.h>
 
-#include "gemv_general.h"
+#include "formats.h"
 #include "gemv_w8.h"
 #include "gemv_w4.h"
 #include "gemv_w4_panel.h"
-#include "generic_nbits.h"
-#include "mfma_block.h"
-#include "mfma_general.h"
-#include "w4a8.h"
-#include "gqa_split.h"
 #include "gqa.h"
 #include "mfma_w4.h"
 #include "mfma_w4_pipe.h"
@@ -909,54 +904,6 @@ bool general_eligible(const Weights& w)
     return (w.K % 8) == 0 && (w.bs % 8) == 0 && (int64_t)w.N * w.nb * w.blob < ((int64_t)1 << 40);
 }
 
-typedef void (*GenGemvFn)(RawLayout, const float*, float*);
-template <size_t... I>
-constexpr std::array<GenGemvFn, sizeof...(I)> gen_gemv_table(std::index_sequence<I...>)
-{
-    return {gemv_general_kernel<(int)I + 1>...};
-}
-constexpr auto kGenGemvTable = gen_gemv_table(std::make_index_sequence<16>{});
-
-template <bool B8, size_t... I>
-constexpr std::array<void (*)(RawLayout, const float*, float*, int, int), sizeof...(I)> gen_chunk_table(
-    std::index_sequence<I...>)
-{
-    return {gemv_chunk_kernel<(int)I + 1, B8>...};
-}
-constexpr auto kGenChunk4Table = gen_chunk_table<false>(std::make_index_sequence<16>{});
-constexpr auto kGenChunk8Table = gen_chunk_table<true>(std::make_index_sequence<16>{});
-
-int log2_exact(int v);
-
-// gemv_chunk_kernel: blocks of whole 16-byte chunks of codes, a power of two of them (so that
-// every chunk lies in one block and is 16-byte aligned).
-bool gemv_chunk_fits(const Weights& w)
-{
-    const int chunk = w.bits == 8 ? 16 : 32;
-    return w.bs % chunk == 0 && log2_exact(w.bs / chunk) >= 0;
-}
-
-int launch_gemv_general(const Weights& w, const float* dA, float* dY, int M, hipStream_t stream)
-{
-    if (gemv_chunk_fits(w)) {
-        const int chunk = w.bits == 8 ? 16 : 32, C = (w.K + chunk - 1) / chunk;
-        const int tile = std::min(C, kGenPanelBytes / (M * chunk * (int)sizeof(float)));
-        const auto fn = (w.bits == 8 ? kGenChunk8Table : kGenChunk4Table)[M - 1];
-        hipLaunchKernelGGL(fn, dim3((w.N + kGenChunkRows - 1) / kGenChunkRows), dim3(512),
-                           (size_t)M * tile * chunk * sizeof(float), stream, raw_layout(w), dA, dY,
-                           log2_exact(w.bs / chunk), tile);
-        MS_HIP_CHECK(hipGetLastError());
-        return MS_HIP_OK;
-    }
-    hipLaunchKernelGGL(kGenGemvTable[M - 1], dim3((w.N + kGenRowsPerWg - 1) / kGenRowsPerWg), dim3(256), 0, stream,
-                       raw_layout(w), dA, dY);
-    MS_HIP_CHECK(hipGetLastError());
-    return MS_HIP_OK;
-}
-
-// ---- gemv_w8: 8-bit decode GEMV ------------------------------------------------------------
-// Instantiations [M-1][config][panel slot]: slot 0 stages the activations through
-// registers (up to kGemv8Av float4 per thread), slot 1 in a loop.
 typedef void (*Gemv8Fn)(Gemv8Params);
 template <int M, size_t I>
 constexpr std::array<Gemv8Fn, 2> gemv8_pair()
@@ -979,13 +926,6 @@ const std::array<std::array<Gemv8Fn, 2>, kNumGemv8Configs> kGemv8Table[kGemvMaxM
     gemv8_row<1>(), gemv8_row<2>(), gemv8_row<3>(), gemv8_row<4>(),
 };
 std::atomic<bool> g_gemv8_lds_raised[kGemvMaxM][kNumGemv8Configs][2];
-
-int log2_exact(int v)
-{
-    int l = 0;
-    while ((1 << l) < v) ++l;
-    return (1 << l) == v ? l : -1;
-}
 
 // gemv_w8 takes 8-bit codes with packed or default zero points, M <= 4, a power-of-two
 // block size >= 16, K a multiple of 16, an activation panel that fits LDS, and buffers
@@ -1040,32 +980,6 @@ int launch_gemv_w8(const Weights& w, const Knobs& kn, const float* dA, float* dY
     p.zrb = w.zrb;
     p.lcpb = log2_exact(w.bs / 16);
     hipLaunchKernelGGL(fn, dim3(gemv8_grid(w, ci)), dim3(kGemv8Configs[ci].waves * kWave), lds, stream, p);
-    MS_HIP_CHECK(hipGetLastError());
-    return MS_HIP_OK;
-}
-
-int launch_mfma_general(const Weights& w, const float* dA, float* dY, int M, hipStream_t stream)
-{
-    GenParams p;
-    p.L = raw_layout(w);
-    p.wexp = w.d_wexp;
-    p.a = dA;
-    p.y = dY;
-    p.M = M;
-    p.tiles_m = (M + kGenBM - 1) / kGenBM;
-    p.tiles_n = (w.N + kGenBN - 1) / kGenBN;
-    const int tiles = p.tiles_m * p.tiles_n;
-    hipLaunchKernelGGL(mfma_general_kernel, dim3(((tiles + kXcds - 1) / kXcds) * kXcds), dim3(256), 0, stream, p);
-    MS_HIP_CHECK(hipGetLastError());
-    return MS_HIP_OK;
-}
-
-int launch_generic(const Weights& w, const float* dA, float* dY, int M, hipStream_t stream)
-{
-    const int64_t total = (int64_t)M * w.N;
-    const int64_t grid = (total + 255) / 256;
-    hipLaunchKernelGGL(nbits_generic_kernel, dim3((unsigned)grid), dim3(256), 0, stream, raw_layout(w), dA,
-                       dY, M);
     MS_HIP_CHECK(hipGetLastError());
     return MS_HIP_OK;
 }
@@ -1528,50 +1442,6 @@ int ensure_rb_layout(Weights& w, hipStream_t stream)
     return 1;
 }
 
-// ---- mfma_block: the general formats with block sizes 16, 32, ..., 512 -----------------------
-// Needs a workspace (A's images); where none can be had mfma_general takes the call.
-bool block_eligible(const Weights& w)
-{
-    const int64_t G = ((int64_t)w.nb * w.bs + 63) / 64;
-    return general_eligible(w) && w.bs >= 16 && w.bs <= 512 && (w.bs & (w.bs - 1)) == 0 &&
-           64 * (int64_t)w.nb * w.blob < kPipeFar && 64 * (int64_t)w.nb * 4 < kPipeFar &&
-           2 * G * kBlkImage < kPipeFar;
-}
-
-// Tiles of 64 x 128 from two per CU on (a lone wave on a SIMD issues a VALU instruction in 6 to 7
-// cycles, two of them one in 4), else 32 x 64 with K over the four waves.
-bool block_whole_k(const Weights& w, int M)
-{
-    return (int64_t)((M + 63) / 64) * ((w.N + 127) / 128) >= 2 * device_cus();
-}
-
-struct BlockWs {
-    int G = 0;
-    size_t rexp_off = 0, total = 0;
-};
-
-BlockWs block_ws(const Weights& w, int M)
-{
-    BlockWs L;
-    L.G = (int)(((int64_t)w.nb * w.bs + 63) / 64);
-    L.rexp_off = (size_t)((M + 31) / 32) * L.G * kBlkImage;
-    L.total = L.rexp_off + align256((size_t)M * sizeof(int));
-    return L;
-}
-
-typedef void (*BlockFn)(BlockParams);
-template <bool B8, bool FZ, int BL>
-BlockFn block_fn(bool whole_k)
-{
-    return whole_k ? mfma_block_kernel<B8, FZ, BL, 2, 2, 1> : mfma_block_kernel<B8, FZ, BL, 1, 1, 4>;
-}
-template <bool B8, bool FZ>
-BlockFn block_fn(int bs, bool whole_k)
-{
-    return bs == 16 ? block_fn<B8, FZ, 4>(whole_k) : bs == 32 ? block_fn<B8, FZ, 5>(whole_k)
-           : bs == 64 ? block_fn<B8, FZ, 6>(whole_k) : block_fn<B8, FZ, 7>(whole_k);
-}
-
 // The stream's workspace of at least `bytes`, under block_mu; nullptr while the stream is being
 // captured (a graph may be replayed beside other calls), for the per-thread stream (one value
 // that names many streams), for a fifth stream, and when memory is short.
@@ -1605,38 +1475,17 @@ uint8_t* block_workspace(Weights& w, size_t bytes, hipStream_t stream)
     return b.data;
 }
 
-// Returns -1 when the call is not taken (mfma_general is to take it).
-int launch_mfma_block(Weights& w, const float* dA, float* dY, int M, hipStream_t stream)
+// mfma_block: the general formats with block sizes 16, 32, ..., 512. Needs a workspace (A's
+// images); where none can be had mfma_general takes the call (-1).
+int launch_block(Weights& w, const float* dA, float* dY, int M, hipStream_t stream)
 {
-    if (!block_eligible(w)) return -1;
-    const BlockWs B = block_ws(w, M);
+    const RawLayout L = raw_layout(w);
+    const BlockPlan plan = block_plan(L, M, device_cus());
+    if (!plan.eligible) return -1;
     std::lock_guard<std::mutex> lock(w.block_mu);   // held over both launches: they share the workspace
-    uint8_t* const data = block_workspace(w, B.total, stream);
+    uint8_t* const data = block_workspace(w, plan.bytes, stream);
     if (!data) return -1;
-    const bool whole = block_whole_k(w, M);
-    BlockParams p;
-    p.L = raw_layout(w);
-    p.wexp = w.d_wexp;
-    p.img = data;
-    p.rexp = reinterpret_cast<const int*>(data + B.rexp_off);
-    p.y = dY;
-    p.M = M;
-    p.G = B.G;
-    p.log2bs = log2_exact(w.bs);
-    p.tiles_m = (M + (whole ? 63 : 31)) / (whole ? 64 : 32);
-    p.tiles_n = (w.N + (whole ? 127 : 63)) / (whole ? 128 : 64);
-    const unsigned rows = (unsigned)((M + 32 * kXcds - 1) / (32 * kXcds) * (32 * kXcds));
-    hipLaunchKernelGGL(block_stage_a_kernel, dim3(rows), dim3(256), 0, stream, dA, data,
-                       reinterpret_cast<int*>(data + B.rexp_off), M, w.K, B.G, p.log2bs);
-    MS_HIP_CHECK(hipGetLastError());
-    const bool fz = w.zp_float;
-    const BlockFn fn = w.bits == 8 ? (fz ? block_fn<true, true>(w.bs, whole) : block_fn<true, false>(w.bs, whole))
-                                   : (fz ? block_fn<false, true>(w.bs, whole) : block_fn<false, false>(w.bs, whole));
-    const int lds = (whole ? 4 : 8) * kBlkImage, tiles = p.tiles_m * p.tiles_n;
-    if (lds > 64 * 1024)
-        MS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    hipLaunchKernelGGL(fn, dim3(((tiles + kXcds - 1) / kXcds) * kXcds), dim3(256), lds, stream, p);
-    MS_HIP_CHECK(hipGetLastError());
+    MS_HIP_CHECK(launch_mfma_block(L, w.d_wexp, plan, data, dA, dY, M, stream));
     return MS_HIP_OK;
 }
 
@@ -1699,14 +1548,15 @@ int launch_kernel(Weights& w, const Knobs& kn, KernelId k, const Ws& ws, const f
                   hipStream_t stream, AConv* conv = nullptr, bool may_alloc = true)
 {
     switch (k) {
-        case kGeneric: return launch_generic(w, dA, dY, M, stream);
-        case kGemvGeneral: return launch_gemv_general(w, dA, dY, M, stream);
+        case kGeneric: MS_HIP_CHECK(launch_generic(raw_layout(w), dA, dY, M, stream)); return MS_HIP_OK;
+        case kGemvGeneral: MS_HIP_CHECK(launch_gemv_general(raw_layout(w), dA, dY, M, stream)); return MS_HIP_OK;
         case kMfmaGeneral:
             if (may_alloc) {
-                const int r = launch_mfma_block(w, dA, dY, M, stream);
+                const int r = launch_block(w, dA, dY, M, stream);
                 if (r >= 0) return r;
             }
-            return launch_mfma_general(w, dA, dY, M, stream);
+            MS_HIP_CHECK(launch_mfma_general(raw_layout(w), w.d_wexp, dA, dY, M, stream));
+            return MS_HIP_OK;
         case kGemvW8: return launch_gemv_w8(w, kn, dA, dY, M, stream);
         case kGemv:
         case kPanel: return launch_gemv(w, kn, dA, dY, M, stream);
@@ -1763,137 +1613,6 @@ int enqueue_gemm(Weights& w, const float* dA, float* dY, int M, hipStream_t stre
 }
 
 // ---- W4A8 (the opt-in approximate product) --------------------------------------------------
-enum W4a8KernelId { kW8Gemv = 9, kW8Mfma = 10, kW8Generic = 11 };
-
-// The GEMM's dots are exact while a block's sum stays below 2^24.
-W4a8KernelId w4a8_kernel(const Weights& w, int M)
-{
-    if (w.bits == 4 && w.bs % 32 == 0) {
-        if (M <= 16) return kW8Gemv;
-        if ((int64_t)w.bs * 127 * 15 < (1 << 24)) return kW8Mfma;
-    }
-    return kW8Generic;
-}
-
-// Rows of A per workgroup of the GEMM, in units of 16: the least work on the fullest CU,
-// which runs ceil(workgroups / 256) of them; per 32-code step about 21 VALU instructions for
-// the weights' dequant and the loop, and per unit 12 / spb for the sums and 2 for what of the
-// MFMAs they do not cover.
-int w4a8_nf(const Weights& w, int M)
-{
-    int best = 2;
-    int64_t cost = INT64_MAX;
-    for (int nf : {8, 4, 2}) {
-        const int64_t wgs = (int64_t)((M + 16 * nf - 1) / (16 * nf)) * ((w.N + kW8BN - 1) / kW8BN);
-        const int spb = w.bs / 32;
-        const int64_t c = (wgs + device_cus() - 1) / device_cus() * ((12 + 2 * spb) * nf + 21 * spb);
-        if (c < cost) {
-            cost = c;
-            best = nf;
-        }
-    }
-    return best;
-}
-
-// Workspace of one call. The GEMM: the images of A (w4a8_stage_kernel). The others:
-// activation codes [M][padK] and, 256-byte aligned, their scales [M][nb].
-struct W4a8Layout {
-    int padK = 0, nf = 0, tiles_m = 0, G = 0;
-    size_t sa_off = 0, total = 0;
-};
-
-W4a8Layout w4a8_layout(const Weights& w, int M)
-{
-    W4a8Layout L;
-    L.padK = ((w.nb * w.bs + 31) / 32) * 32;
-    if (w4a8_kernel(w, M) == kW8Mfma) {
-        L.nf = w4a8_nf(w, M);
-        L.tiles_m = (M + 16 * L.nf - 1) / (16 * L.nf);
-        L.G = (L.padK / 32 + 3) / 4;
-        L.total = (size_t)L.tiles_m * L.G * w4a8_image_bytes(L.nf);
-        return L;
-    }
-    L.sa_off = align256((size_t)M * L.padK);
-    L.total = L.sa_off + align256((size_t)M * w.nb * sizeof(float));
-    return L;
-}
-
-int w4a8_grid(const Weights& w, int M, W4a8KernelId k)
-{
-    if (k == kW8Gemv) return (w.N + kW8RowsPerWg - 1) / kW8RowsPerWg;
-    if (k == kW8Mfma) {
-        const int tiles = w4a8_layout(w, M).tiles_m * ((w.N + kW8BN - 1) / kW8BN);
-        return ((tiles + kXcds - 1) / kXcds) * kXcds;
-    }
-    return (int)(((int64_t)M * w.N + 255) / 256);
-}
-
-typedef void (*W8MfmaFn)(W4a8MfmaParams);
-template <int NF>
-W8MfmaFn w8_mfma_fn(int spb)
-{
-    return spb == 1       ? mfma_w4a8_kernel<NF, 1>
-           : spb == 2     ? mfma_w4a8_kernel<NF, 2>
-           : spb % 4 == 0 ? mfma_w4a8_kernel<NF, 4>
-                          : mfma_w4a8_kernel<NF, 0>;
-}
-
-typedef void (*W8GemvFn)(RawLayout, W4a8Args, float*);
-template <size_t... I>
-constexpr std::array<W8GemvFn, sizeof...(I)> w8_gemv_table(std::index_sequence<I...>)
-{
-    return {gemv_w4a8_kernel<(int)I + 1>...};
-}
-constexpr auto kW8GemvTable = w8_gemv_table(std::make_index_sequence<16>{});
-
-int launch_w4a8(const Weights& w, const Ws& ws, const float* dA, float* dY, int M, hipStream_t stream)
-{
-    const W4a8Layout Lw = w4a8_layout(w, M);
-    const RawLayout L = raw_layout(w);
-    const W4a8KernelId k = w4a8_kernel(w, M);
-    const int grid = w4a8_grid(w, M, k);
-    if (k == kW8Mfma) {
-        const int64_t threads = (int64_t)M * w.nb * 4;
-        hipLaunchKernelGGL(w4a8_stage_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, dA,
-                           ws.data, M, w.K, w.bs, w.nb, Lw.G, Lw.nf);
-        MS_HIP_CHECK(hipGetLastError());
-        W4a8MfmaParams p;
-        p.L = L;
-        p.img = ws.data;
-        p.y = dY;
-        p.M = M;
-        p.G = Lw.G;
-        p.tiles_m = Lw.tiles_m;
-        p.tiles_n = (w.N + kW8BN - 1) / kW8BN;
-        const int spb = w.bs / 32;
-        const W8MfmaFn fn = Lw.nf == 2 ? w8_mfma_fn<2>(spb) : Lw.nf == 4 ? w8_mfma_fn<4>(spb) : w8_mfma_fn<8>(spb);
-        const int lds = 2 * w4a8_image_bytes(Lw.nf);
-        if (lds > 64 * 1024)
-            MS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             lds));
-        hipLaunchKernelGGL(fn, dim3(grid), dim3(256), lds, stream, p);
-        MS_HIP_CHECK(hipGetLastError());
-        return MS_HIP_OK;
-    }
-    int8_t* aq = reinterpret_cast<int8_t*>(ws.data);
-    float* sa = reinterpret_cast<float*>(ws.data + Lw.sa_off);
-    const int64_t threads = (int64_t)M * w.nb * 8;
-    hipLaunchKernelGGL(w4a8_quantize_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, dA, aq,
-                       sa, M, w.K, w.bs, w.nb, Lw.padK);
-    MS_HIP_CHECK(hipGetLastError());
-    W4a8Args A;
-    A.aq = aq;
-    A.sa = sa;
-    A.M = M;
-    A.padK = Lw.padK;
-    if (k == kW8Gemv)
-        hipLaunchKernelGGL(kW8GemvTable[M - 1], dim3(grid), dim3(256), 0, stream, L, A, dY);
-    else
-        hipLaunchKernelGGL(w4a8_generic_kernel, dim3(grid), dim3(256), 0, stream, L, A, dY);
-    MS_HIP_CHECK(hipGetLastError());
-    return MS_HIP_OK;
-}
-
 int enqueue_w4a8(Weights& w, const float* dA, float* dY, int M, hipStream_t stream)
 {
     if (w.zp_float)
@@ -1903,13 +1622,16 @@ int enqueue_w4a8(Weights& w, const float* dA, float* dY, int M, hipStream_t stre
     int st = check_call(dA, dY, M);
     if (st || M == 0) return st;
     Ws ws;
-    const int r = ensure_ws(w, w4a8_layout(w, M).total, 0, stream, &ws);
+    const RawLayout L = raw_layout(w);
+    const W4a8Plan plan = w4a8_plan(L, M, device_cus());
+    const int r = ensure_ws(w, plan.bytes, 0, stream, &ws);
     if (r < 0) return fail(MS_HIP_ERR_HIP, "[ms_hip] workspace allocation failed: %s", hipGetErrorString(hipGetLastError()));
     if (r == 0)
         return fail(MS_HIP_ERR_UNSUPPORTED,
                     "[ms_hip] W4A8 needs the handle's workspace, which cannot grow under stream capture: "
                     "make one call of this size outside the capture first");
-    return launch_w4a8(w, ws, dA, dY, M, stream);
+    MS_HIP_CHECK(launch_w4a8(L, plan, ws.data, dA, dY, M, stream));
+    return MS_HIP_OK;
 }
 
 int check_impl(int N, int K, int bits, int bs, int64_t b_len, int64_t scales_len, int zp_kind, int64_t zp_len,
@@ -2019,9 +1741,7 @@ int finish_create(Weights* w, int st, void** out_handle)
 {
     if (!st) st = check_pipe_scales(*w);
     if (!st && w->d_wexp) {   // row exponents of the general GEMM
-        hipLaunchKernelGGL(weight_row_exponent_kernel, dim3((w->N + 255) / 256), dim3(256), 0, nullptr, raw_layout(*w),
-                           w->d_wexp);
-        hipError_t e = hipGetLastError();
+        hipError_t e = launch_row_exponents(raw_layout(*w), w->d_wexp, nullptr);
         if (e == hipSuccess) e = hipDeviceSynchronize();
         if (e != hipSuccess) st = fail(MS_HIP_ERR_HIP, "[ms_hip] weight exponents failed: %s", hipGetErrorString(e));
     }
@@ -2823,9 +2543,9 @@ int ms_hip_nbits_launch_info_w4a8(void* handle, int M, int* kernel_id, int* grid
     if (!w) return fail(MS_HIP_ERR_INVALID, "[ms_hip] invalid weights handle");
     if (M <= 0) return fail(MS_HIP_ERR_INVALID, "[ms_hip] M must be positive; got %d", M);
     if (w->zp_float) return fail(MS_HIP_ERR_UNSUPPORTED, "[ms_hip] W4A8 takes packed or default zero points");
-    const W4a8KernelId k = w4a8_kernel(*w, M);
-    if (kernel_id) *kernel_id = (int)k;
-    if (grid) *grid = w4a8_grid(*w, M, k);
+    const W4a8Plan plan = w4a8_plan(raw_layout(*w), M, device_cus());
+    if (kernel_id) *kernel_id = (int)plan.kernel;
+    if (grid) *grid = plan.grid;
     return MS_HIP_OK;
 }
 
@@ -2876,10 +2596,7 @@ int ms_hip_nbits_dequant_dev(void* handle, float* dW, void* stream)
     Weights* w = from_handle(handle);
     if (!w) return fail(MS_HIP_ERR_INVALID, "[ms_hip] invalid weights handle");
     if (!dW) return fail(MS_HIP_ERR_INVALID, "[ms_hip] null output pointer");
-    const int64_t total = (int64_t)w->N * w->K;
-    hipLaunchKernelGGL(nbits_dequant_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), raw_layout(*w), dW);
-    MS_HIP_CHECK(hipGetLastError());
+    MS_HIP_CHECK(launch_dequant(raw_layout(*w), dW, static_cast<hipStream_t>(stream)));
     return MS_HIP_OK;
 }
 
@@ -2994,10 +2711,10 @@ int ms_hip_nbits_launch_info(void* handle, int M, int* kernel_id, int* lanes_per
     switch (kid) {
         case kGeneric: gr = (int)(((int64_t)M * w->N + 255) / 256); break;
         case kGemvGeneral: {
-            const int rows = gemv_chunk_fits(*w) ? kGenChunkRows : kGenRowsPerWg;
-            gr = (w->N + rows - 1) / rows;
+            const LaunchShape shape = gemv_general_shape(raw_layout(*w));
+            gr = shape.grid;
+            bl = shape.block;
             G = 16;
-            if (gemv_chunk_fits(*w)) bl = 512;
             break;
         }
         case kGemvW8: {
@@ -3008,10 +2725,8 @@ int ms_hip_nbits_launch_info(void* handle, int M, int* kernel_id, int* lanes_per
             break;
         }
         case kMfmaGeneral:
-            gr = ((M + kGenBM - 1) / kGenBM) * ((w->N + kGenBN - 1) / kGenBN);
-            if (block_eligible(*w))
-                gr = block_whole_k(*w, M) ? ((M + 63) / 64) * ((w->N + 127) / 128) : ((M + 31) / 32) * ((w->N + 63) / 64);
-            gr = ((gr + kXcds - 1) / kXcds) * kXcds;
+            gr = mfma_general_grid(raw_layout(*w), M);
+            if (const BlockPlan b = block_plan(raw_layout(*w), M, device_cus()); b.eligible) gr = b.grid;
             break;
         case kSkinny: gr = ((w->N + kSkinnyRows - 1) / kSkinnyRows) * skinny_ksw(*w, kn); break;
         case kGemv: {
@@ -3191,8 +2906,7 @@ bool gqa_split_fits(const ms_hip_gqa_desc& d)
     const int64_t total = (int64_t)d.past_seq + d.kv_seq;
     const int64_t visible = d.local_window_size >= 0 ? std::min(total, (int64_t)d.local_window_size + d.q_seq) : total;
     return d.q_seq > 8 && (D == 64 || D == 96 || D == 128) && d.batch > 0 && visible >= (D == 64 ? 192 : 128) && total <= 2 * visible &&
-           d.scale >= 0.0f && d.scale <= 65536.0f && gqa_split_chunks(total) * (int64_t)(512 * D) < kPipeFar &&
-           (int64_t)d.batch * d.kv_num_heads * gqa_split_chunks(total) < (1 << 30);
+           d.scale >= 0.0f && d.scale <= 65536.0f && gqa_split_sizes(d.batch, d.kv_num_heads, total, D);
 }
 
 GqaPlan gqa_plan(const ms_hip_gqa_desc& d, int64_t ws_avail, bool split_ok = true)
@@ -3200,13 +2914,12 @@ GqaPlan gqa_plan(const ms_hip_gqa_desc& d, int64_t ws_avail, bool split_ok = tru
     GqaPlan pl;
     const int D = d.head_dim;
     if (split_ok && gqa_split_fits(d)) {
-        const int64_t ws = gqa_split_ws_bytes((int64_t)d.batch * d.kv_num_heads, (int64_t)d.past_seq + d.kv_seq, D);
+        const int64_t ws = gqa_split_bytes((int64_t)d.batch * d.kv_num_heads, (int64_t)d.past_seq + d.kv_seq, D);
         if (ws_avail < 0 || ws <= ws_avail) {
             // 128 queries per workgroup while that still gives every CU one, else 64 (a block of
             // 64 halves a short launch's waves, and its idle CUs)
             const int64_t wg = (int64_t)d.batch * d.num_heads * ((d.q_seq + 127) / 128);
             pl.split_waves = wg >= 256 ? 4 : 2;
-            pl.lds = (size_t)1024 * D;
             pl.ws_bytes = ws;
             return pl;
         }
@@ -3259,32 +2972,6 @@ GqaPlan gqa_plan(const ms_hip_gqa_desc& d, int64_t ws_avail, bool split_ok = tru
         pl.lds = ((size_t)D + std::max(kGqaThreads, D) + (size_t)total) * sizeof(float);
     }
     return pl;
-}
-
-template <int D, int NW>
-int launch_gqa_split_attention(const GqaArgs& p, const GqaPlan& pl, const GqaSplitWs& w, hipStream_t s)
-{
-    const int64_t grid = gqa_split_grid(p.B * p.kvH, p.H / p.kvH, (p.Sq + 32 * NW - 1) / (32 * NW));
-    if (pl.lds >= 64 * 1024)   // with the kernel's few static bytes above 64 KB
-        MS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(gqa_split_kernel<D, NW>),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.lds));
-    hipLaunchKernelGGL((gqa_split_kernel<D, NW>), dim3((unsigned)grid), dim3(128 * NW), pl.lds, s, p, w);
-    MS_HIP_CHECK(hipGetLastError());
-    return MS_HIP_OK;
-}
-
-template <int D>
-int launch_gqa_split(const GqaArgs& p, const GqaPlan& pl, void* workspace, hipStream_t s)
-{
-    const int units = p.B * p.kvH, nch = gqa_split_chunks(p.total);
-    GqaSplitWs w;
-    w.img = static_cast<uint8_t*>(workspace);
-    w.exps = reinterpret_cast<int*>(w.img + (int64_t)units * nch * (512 * D));
-    w.nch = nch;
-    hipLaunchKernelGGL(gqa_split_kv_kernel<D>, dim3((unsigned)(2 * units * nch)), dim3(256), 0, s, p, w);
-    MS_HIP_CHECK(hipGetLastError());
-    return pl.split_waves == 4 ? launch_gqa_split_attention<D, 4>(p, pl, w, s)
-                               : launch_gqa_split_attention<D, 2>(p, pl, w, s);
 }
 
 }  // namespace
@@ -3393,11 +3080,8 @@ int ms_hip_gqa(const ms_hip_gqa_desc* d, const float* dQ, const float* dK, const
                                              (reinterpret_cast<uintptr_t>(dWorkspace) & 15) == 0)
                                   : GqaPlan{};
     if (plan.split_waves) {
-        switch (p.D) {
-            case 64: return launch_gqa_split<64>(p, plan, dWorkspace, s);
-            case 96: return launch_gqa_split<96>(p, plan, dWorkspace, s);
-            default: return launch_gqa_split<128>(p, plan, dWorkspace, s);
-        }
+        MS_HIP_CHECK(launch_gqa_split(p, plan.split_waves, dWorkspace, s));
+        return MS_HIP_OK;
     }
     if (p.Skv > 0 && !plan.grouped) {   // the grouped kernel writes the new rows itself
         const int threads = std::min(256, ((p.D + 63) / 64) * 64);

@@ -25,7 +25,7 @@
 //                          per output, the definition above as written
 #pragma once
 #include "generic_nbits.h"
-#include "mfma_w4_pipe.h"
+#include "mfma_device.h"
 
 namespace msnb {
 
