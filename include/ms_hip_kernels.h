@@ -156,7 +156,14 @@ int ms_hip_nbits_gemm(void* handle, const float* a_host, float* y_host, int M);
  * If they do, or a hand-off between the two halves of a split tile does not
  * complete within its bound, the kernel records it in the handle's error word and
  * the output of that call is not valid: the next call on the handle (or
- * ms_hip_nbits_device_error) returns MS_HIP_ERR_HIP and clears the record. */
+ * ms_hip_nbits_device_error) returns MS_HIP_ERR_HIP and clears the record.
+ * The general formats (float zero points, 8-bit codes and block sizes the 4-bit
+ * kernels do not take) with a block size of 16, 32, ..., 512 stage A at M > 16 as two
+ * fp16 halves and block sums, 4.5 bytes per activation, in a buffer of the handle's
+ * own, freed with it. Their eager calls on one handle may overlap on several streams
+ * (from the second stream on a call waits for the one before it on the device); a graph that holds such a call
+ * must not be replayed beside other calls on the handle, and a stream is synchronised
+ * after such a call before it is destroyed. */
 int ms_hip_nbits_gemm_dev(void* handle, const float* dA, float* dY, int M, void* stream);
 
 /* ms_hip_nbits_gemm_dev with fp16 activations (q4f16 exports): dA16 is [M,K] fp16,
@@ -168,14 +175,16 @@ int ms_hip_nbits_gemm_dev_f16(void* handle, const void* dA16, float* dY, int M, 
 /* Allocation-free form of ms_hip_nbits_gemm_dev, for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc). No counterpart in the reference. Same arguments, kernels and
- * results as ms_hip_nbits_gemm_dev, with one exception: a call that
+ * results as ms_hip_nbits_gemm_dev, with two exceptions. A call that
  * ms_hip_nbits_gemm_dev would run on mfma_w4_rb (M > 16 prefill) needs the handle's
  * chunk-major scale copy, which the first such eager call builds (an allocation); until
  * one has, this entry runs the call on mfma_w4 (the exact-scale prefill kernel: the same
- * 2e-3 relative Frobenius bar, not bit-identical). The workspace comes from a fixed scratch array
+ * 2e-3 relative Frobenius bar, not bit-identical). And a general-format call of M > 16
+ * whose images of A (see ms_hip_nbits_gemm_dev) exceed the scratch runs the general
+ * kernel that needs none. The workspace comes from a fixed scratch array
  * that the library holds on each GPU it runs on until the process ends (96 MiB of
- * data and 64 Ki counters; enough for M = 2048 on the Llama-2-7B MLP shapes). A call
- * that needs more returns MS_HIP_ERR_INVALID without launching anything. Every call
+ * data and 64 Ki counters; enough for M = 2048 on the Llama-2-7B MLP shapes). Any other
+ * call that needs more returns MS_HIP_ERR_INVALID without launching anything. Every call
  * on one GPU shares that GPU's scratch: calls that overlap on one GPU (other streams,
  * other threads) race, and must not be made. The calling thread's current device must
  * be the handle's. */
@@ -326,7 +335,8 @@ int ms_hip_sync(void);
  *   5 skinny_w4, 6 mfma_w4_rb, 7 gemv_general, 8 mfma_general, 12 gemv_w8 (9-11 are
  *   the W4A8 kernels of ms_hip_nbits_launch_info_w4a8); lanes_per_row is the
  *   lanes per weight row of the
- *   GEMV kernels, the output tile width of mfma_w4_rb, 0 otherwise. */
+ *   GEMV kernels, the output tile width of mfma_w4_rb, and under mfma_general that of
+ *   the kernel with staged images of A (64 or 128) where it takes the call; 0 otherwise. */
 /* ms_hip_nbits_batch_launch_info: what the first launch of a batch call with these
  * handles and activations would be: `calls` = how many of the leading calls it
  * serves, then as ms_hip_nbits_launch_info. */

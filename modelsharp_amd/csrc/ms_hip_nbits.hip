@@ -231,16 +231,20 @@ struct Weights {
     uint8_t* d_zp = nullptr;
     float* d_zpf = nullptr;     // float zero points [N * nb]
     int* d_wexp = nullptr;      // general formats: row exponents of the weights [N]
-    // mfma_block's workspaces, one per stream that has called (the format's calls may overlap on
-    // several streams: mfma_general, which further streams and captured calls get, needs none)
-    struct BlockSlot {
-        hipStream_t stream = nullptr;
-        uint8_t* data = nullptr;
-        size_t bytes = 0;
-    };
+    // mfma_block's workspace (A's images), guarded by block_mu and grown by eager calls. Calls on
+    // one stream follow each other. From a call on a second stream on the handle orders its eager
+    // calls by an event behind each (3 us a call, which the others do not pay), in a new buffer,
+    // as the first may still be in use. (Streams are told apart by their handles: one destroyed
+    // with such a call in flight and another made at its address pass for one stream, so the
+    // header asks for a synchronisation before the destruction.) A captured call takes the
+    // buffer as it is; one that a graph may hold is kept until the handle goes.
     std::mutex block_mu;
-    std::array<BlockSlot, 4> block_slots;
-    int block_used = 0;
+    uint8_t* d_block = nullptr;
+    size_t block_bytes = 0;
+    hipStream_t block_stream = nullptr;
+    hipEvent_t block_done = nullptr;   // set from the second stream on
+    bool block_captured = false;
+    std::vector<uint8_t*> block_kept;
     // mfma_w4_rb's chunk-major scales / zero points [K / 128][N][4], built by the first
     // eager call that takes it (rb_ready then 1; guarded by ws_mu)
     uint32_t* d_sz4 = nullptr;
@@ -333,11 +337,9 @@ void free_weights(Weights& w)
     if (w.d_zp) (void)hipFree(w.d_zp);
     if (w.d_zpf) (void)hipFree(w.d_zpf);
     if (w.d_wexp) (void)hipFree(w.d_wexp);
-    for (auto& b : w.block_slots) {
-        if (b.data) (void)hipFree(b.data);
-        b.data = nullptr;
-        b.bytes = 0;
-    }
+    if (w.d_block) (void)hipFree(w.d_block);
+    for (uint8_t* p : w.block_kept) (void)hipFree(p);
+    if (w.block_done) (void)hipEventDestroy(w.block_done);
     if (w.d_stage) (void)hipFree(w.d_stage);
     if (w.h_stage) (void)hipHostFree(w.h_stage);
     if (w.h_err) (void)hipHostFree(w.h_err);
@@ -349,6 +351,10 @@ void free_weights(Weights& w)
     w.d_zp = nullptr;
     w.d_zpf = nullptr;
     w.d_wexp = nullptr;
+    w.d_block = nullptr;
+    w.block_bytes = 0;
+    w.block_kept.clear();
+    w.block_done = nullptr;
     w.d_stage = nullptr;
     w.stage_bytes = 0;
     w.h_stage = nullptr;
@@ -1442,50 +1448,58 @@ int ensure_rb_layout(Weights& w, hipStream_t stream)
     return 1;
 }
 
-// The stream's workspace of at least `bytes`, under block_mu; nullptr while the stream is being
-// captured (a graph may be replayed beside other calls), for the per-thread stream (one value
-// that names many streams), for a fifth stream, and when memory is short.
+// The handle's block workspace of at least `bytes` for an eager call on `stream`, under
+// block_mu, the stream behind the workspace's last eager use; nullptr when memory is short.
 uint8_t* block_workspace(Weights& w, size_t bytes, hipStream_t stream)
 {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (stream == hipStreamPerThread || hipStreamIsCapturing(stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
-        (void)hipGetLastError();
-        return nullptr;
+    if (w.block_done) {
+        if (hipStreamWaitEvent(stream, w.block_done, 0) != hipSuccess) return nullptr;
+    } else if (stream == hipStreamPerThread || (w.d_block && stream != w.block_stream)) {
+        if (hipEventCreateWithFlags(&w.block_done, hipEventDisableTiming) != hipSuccess) return nullptr;
+        if (w.d_block) w.block_kept.push_back(w.d_block);
+        w.d_block = nullptr;
+        w.block_bytes = 0;
     }
-    int i = 0;
-    while (i < w.block_used && w.block_slots[i].stream != stream) ++i;
-    if (i == (int)w.block_slots.size()) return nullptr;
-    auto& b = w.block_slots[i];
-    if (b.bytes < bytes) {
-        // earlier launches on this stream may still use the old buffer
-        if (b.data && (hipStreamSynchronize(stream) != hipSuccess || hipFree(b.data) != hipSuccess)) return nullptr;
-        b.data = nullptr;
-        b.bytes = 0;
-        if (hipMalloc(&b.data, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            b.data = nullptr;
+    w.block_stream = stream;
+    if (w.block_bytes < bytes) {
+        // earlier calls may still use the old buffer
+        if (w.d_block && w.block_captured) {
+            w.block_kept.push_back(w.d_block);
+        } else if (w.d_block) {
+            if (hipStreamSynchronize(stream) != hipSuccess) return nullptr;
+            (void)hipFree(w.d_block);
+        }
+        w.d_block = nullptr;
+        w.block_bytes = 0;
+        w.block_captured = false;
+        if (hipMalloc(&w.d_block, bytes) != hipSuccess) {
+            w.d_block = nullptr;
             return nullptr;
         }
-        b.bytes = bytes;
+        w.block_bytes = bytes;
     }
-    if (i == w.block_used) {
-        b.stream = stream;
-        ++w.block_used;
-    }
-    return b.data;
+    return w.d_block;
 }
 
 // mfma_block: the general formats with block sizes 16, 32, ..., 512. Needs a workspace (A's
-// images); where none can be had mfma_general takes the call (-1).
+// images); where none can be had (a captured call larger than the eager ones before it, memory
+// short) mfma_general takes the call (-1).
 int launch_block(Weights& w, const float* dA, float* dY, int M, hipStream_t stream)
 {
     const RawLayout L = raw_layout(w);
     const BlockPlan plan = block_plan(L, M, device_cus());
     if (!plan.eligible) return -1;
     std::lock_guard<std::mutex> lock(w.block_mu);   // held over both launches: they share the workspace
-    uint8_t* const data = block_workspace(w, plan.bytes, stream);
-    if (!data) return -1;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    const bool eager = hipStreamIsCapturing(stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
+    uint8_t* const data = eager ? block_workspace(w, plan.bytes, stream) : w.block_bytes >= plan.bytes ? w.d_block : nullptr;
+    if (!data) {
+        (void)hipGetLastError();
+        return -1;
+    }
+    w.block_captured |= !eager;
     MS_HIP_CHECK(launch_mfma_block(L, w.d_wexp, plan, data, dA, dY, M, stream));
+    if (eager && w.block_done) MS_HIP_CHECK(hipEventRecord(w.block_done, stream));
     return MS_HIP_OK;
 }
 
@@ -1545,16 +1559,13 @@ KernelId workspace_free_kernel(const Weights& w, const Knobs& kn, int M)
 }
 
 int launch_kernel(Weights& w, const Knobs& kn, KernelId k, const Ws& ws, const float* dA, float* dY, int M,
-                  hipStream_t stream, AConv* conv = nullptr, bool may_alloc = true)
+                  hipStream_t stream, AConv* conv = nullptr)
 {
     switch (k) {
         case kGeneric: MS_HIP_CHECK(launch_generic(raw_layout(w), dA, dY, M, stream)); return MS_HIP_OK;
         case kGemvGeneral: MS_HIP_CHECK(launch_gemv_general(raw_layout(w), dA, dY, M, stream)); return MS_HIP_OK;
         case kMfmaGeneral:
-            if (may_alloc) {
-                const int r = launch_block(w, dA, dY, M, stream);
-                if (r >= 0) return r;
-            }
+            if (const int r = launch_block(w, dA, dY, M, stream); r >= 0) return r;
             MS_HIP_CHECK(launch_mfma_general(raw_layout(w), w.d_wexp, dA, dY, M, stream));
             return MS_HIP_OK;
         case kGemvW8: return launch_gemv_w8(w, kn, dA, dY, M, stream);
@@ -2078,6 +2089,8 @@ int ms_hip_nbits_gemm_dev_noalloc(void* handle, const float* dA, float* dY, int 
     if ((st = resolve_rb(*w, kn, &k, M, s, false))) return st;
     size_t need_d = 0, need_c = 0;
     workspace_need(*w, kn, k, M, &need_d, &need_c);
+    const BlockPlan block = k == kMfmaGeneral ? block_plan(raw_layout(*w), M, device_cus()) : BlockPlan{};
+    if (block.eligible && block.bytes <= kScratchDataBytes) need_d = block.bytes;
     if (need_d > kScratchDataBytes || need_c > kScratchCntInts)
         return fail(MS_HIP_ERR_INVALID,
                     "[ms_hip] this call (M=%d, N=%d, K=%d) needs %zu bytes and %zu counters of workspace; the "
@@ -2101,7 +2114,12 @@ int ms_hip_nbits_gemm_dev_noalloc(void* handle, const float* dA, float* dY, int 
         // at zero (a fill kernel, which a captured graph can hold).
         if ((st = zero_ints(ws.cnt, (int64_t)need_c, s))) return st;
     }
-    return launch_kernel(*w, kn, k, ws, dA, dY, M, s, nullptr, false);
+    if (k == kMfmaGeneral) {   // mfma_block where the scratch holds A's images, as the eager call; else mfma_general
+        MS_HIP_CHECK(ws.data ? launch_mfma_block(raw_layout(*w), w->d_wexp, block, ws.data, dA, dY, M, s)
+                             : launch_mfma_general(raw_layout(*w), w->d_wexp, dA, dY, M, s));
+        return MS_HIP_OK;
+    }
+    return launch_kernel(*w, kn, k, ws, dA, dY, M, s);
 }
 
 int ms_hip_nbits_device_error(void* handle)
@@ -2726,7 +2744,10 @@ int ms_hip_nbits_launch_info(void* handle, int M, int* kernel_id, int* lanes_per
         }
         case kMfmaGeneral:
             gr = mfma_general_grid(raw_layout(*w), M);
-            if (const BlockPlan b = block_plan(raw_layout(*w), M, device_cus()); b.eligible) gr = b.grid;
+            if (const BlockPlan b = block_plan(raw_layout(*w), M, device_cus()); b.eligible) {
+                gr = b.grid;
+                G = b.whole_k ? 128 : 64;   // reported as the tile width
+            }
             break;
         case kSkinny: gr = ((w->N + kSkinnyRows - 1) / kSkinnyRows) * skinny_ksw(*w, kn); break;
         case kGemv: {

@@ -585,3 +585,110 @@ def test_chunk_gemv(gpu, M, bits, K):
     kernel, _ = check_against_oracle(w, a, b, s, None, zpf, op, f"chunk bits={bits} K={K} M={M}")
     assert kernel == "gemv_general"
     w.close()
+
+
+@pytest.mark.parametrize("fzp,op", [(True, Op("b4_bs64", 1000, 200, 64, True)), (False, Op("b4_bs16", 1024, 300, 16, True)),
+                                    (True, Op("b8_bs32", 520, 130, 32, True, bits=8))], ids=lambda v: getattr(v, "name", str(v)))
+def test_block_gemm_is_one_kernel_on_every_route(gpu, op, fzp):
+    """mfma_block's products are the same bits from the eager entry on any of six streams, from
+    the allocation-free entry (before and after the eager call) and from a graph captured after
+    an eager call, replayed with eager work between and after a larger eager call has grown the
+    workspace. A graph captured before any eager call stays within the general kernel's bound."""
+    import torch
+    M = 40
+    b, s, z = workloads.make_weights(op, seed=op.K + M)
+    zpf = float_zero_points(op, seed=op.N + M) if fzp else None
+    z = None if fzp else z
+    a = workloads.make_activations(M, op.K, seed=M, kind="rmsnorm")
+    W = oracle.dequant_weights(b, s, z, op.N, op.K, op.bits, op.block_size, zp_float=zpf)
+    ref = oracle.matmul_nbits(a, b, s, z, op.N, op.K, op.bits, op.block_size, zp_float=zpf)
+    allowed = (4 * gamma2(op.K) + 2.0 ** -20) * dot_abs(a, W) + 2.0 ** -30 * (
+        np.max(np.abs(a), axis=1, keepdims=True).astype(np.float64) * np.abs(W).sum(axis=1)[None, :])
+    w = native.NBitsWeights(b, s, zpf if fzp else z, op.N, op.K, op.bits, op.block_size)
+    dA = torch.from_numpy(a).cuda()
+    dA2 = torch.from_numpy(workloads.make_activations(200, op.K, seed=5)).cuda()
+    dY2 = torch.zeros((200, op.N), device="cuda")
+
+    def run(call, stream=None):
+        y = torch.full((M, op.N), float("nan"), device="cuda")
+        torch.cuda.synchronize()
+        call(dA.data_ptr(), y.data_ptr(), M, stream)
+        torch.cuda.synchronize()
+        return y.cpu().numpy()
+
+    def captured():
+        y = torch.zeros((M, op.N), device="cuda")
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            w.gemm_dev(dA.data_ptr(), y.data_ptr(), M, torch.cuda.current_stream().cuda_stream)
+        return g, y
+
+    def replay(g, y):
+        y.fill_(float("nan"))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        return y.cpu().numpy()
+
+    log(f"block routes {op.name}")
+    first = run(w.gemm_dev_noalloc)
+    assert_within(replay(*captured()), ref, allowed, "captured before an eager call")
+    eager = run(w.gemm_dev)
+    assert_within(eager, ref, allowed, "eager")
+    assert np.array_equal(first, eager) and np.array_equal(run(w.gemm_dev_noalloc), eager)
+    for i, st in enumerate([torch.cuda.Stream() for _ in range(6)]):
+        assert np.array_equal(run(w.gemm_dev, st.cuda_stream), eager), f"stream {i}"
+    g, y = captured()
+    for rows in (20, 40, 200, 200):   # the third grows the workspace: the graph's stays
+        assert np.array_equal(replay(g, y), eager), f"replay before an eager call of {rows} rows"
+        w.gemm_dev(dA2.data_ptr(), dY2.data_ptr(), rows)
+    assert np.array_equal(replay(g, y), eager)
+    assert w.launch_info(M)["lanes_per_row"] == 64   # mfma_block's tiles of 32 x 64
+    w.close()
+
+
+def test_block_gemm_calls_on_two_streams(gpu):
+    """Eager calls on one handle from two streams, enqueued in turn without a wait between them:
+    every call's output is its own input's product."""
+    import torch
+    op, M = Op("b4_bs64", 2048, 1500, 64, True), 96
+    b, s, _ = workloads.make_weights(op, seed=3)
+    w = native.NBitsWeights(b, s, float_zero_points(op, seed=4), op.N, op.K, op.bits, op.block_size)
+    dA = [torch.from_numpy(workloads.make_activations(M, op.K, seed=i)).cuda() for i in range(2)]
+    want = [torch.zeros((M, op.N), device="cuda") for _ in range(2)]
+    for i in range(2):
+        w.gemm_dev(dA[i].data_ptr(), want[i].data_ptr(), M)
+        torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    got = [[torch.zeros((M, op.N), device="cuda") for _ in range(8)] for _ in range(2)]
+    torch.cuda.synchronize()
+    for r in range(8):
+        for i in range(2):
+            w.gemm_dev(dA[i].data_ptr(), got[i][r].data_ptr(), M, streams[i].cuda_stream)
+    torch.cuda.synchronize()
+    for i in range(2):
+        for r in range(8):
+            assert torch.equal(got[i][r], want[i]), f"stream {i} call {r}"
+    w.close()
+
+
+def test_block_gemm_beyond_the_allocation_free_scratch(gpu):
+    """Images larger than the allocation-free entry's scratch (96 MiB): the workspace-free
+    general kernel takes the call, as the header says."""
+    import torch
+    op, M = Op("b4_bs64", 8192, 33, 64, True), 2800
+    b, s, _ = workloads.make_weights(op, seed=3)
+    zpf = float_zero_points(op, seed=4)
+    a = workloads.make_activations(M, op.K, seed=6)
+    w = native.NBitsWeights(b, s, zpf, op.N, op.K, op.bits, op.block_size)
+    dA = torch.from_numpy(a).cuda()
+    y = torch.full((M, op.N), float("nan"), device="cuda")
+    w.gemm_dev_noalloc(dA.data_ptr(), y.data_ptr(), M, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    rows = np.arange(0, M, 31)
+    ref = oracle.matmul_nbits(a[rows], b, s, None, op.N, op.K, 4, 64, zp_float=zpf)
+    W = oracle.dequant_weights(b, s, None, op.N, op.K, 4, 64, zp_float=zpf)
+    allowed = (4 * gamma2(op.K) + 2.0 ** -20) * dot_abs(a[rows], W) + 2.0 ** -30 * (
+        np.max(np.abs(a[rows]), axis=1, keepdims=True).astype(np.float64) * np.abs(W).sum(axis=1)[None, :])
+    assert_within(y.cpu().numpy()[rows], ref, allowed, "beyond the scratch")
+    w.close()
