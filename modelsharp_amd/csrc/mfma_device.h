@@ -54,17 +54,28 @@ typedef __attribute__((address_space(3))) uint8_t lds_byte_t;
 __device__ __forceinline__ uint32_t lds_address(const void* p) { return (uint32_t)(uintptr_t)(lds_byte_t*)p; }
 
 // buffer -> LDS loads: lane i's bytes land at LDS m0 + 16*i (x4) or m0 + 4*i (ushort).
+// The s_nop keeps the wait states that the compiler does not insert before inline asm: one
+// between a write of m0 and the load, five between a vector instruction's write of a scalar
+// operand (a resource reloaded from a spill by v_readlane) and the load. A kernel whose scalar
+// operands are all written by scalar instructions takes one (NOP 0): five cost mfma_w4_pipe 1%
+// (M=512, K=3584 MLP: 332 -> 337 us). test_lds_load_wait_states.py reads both off the built code.
+template <int NOP = 4>
 __device__ __forceinline__ void lds_load16(__amdgpu_buffer_rsrc_t r, int voff, int soff, uint32_t m0v)
 {
-    asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff), "{m0}"(m0v) : "memory");
+    asm volatile("s_nop %4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff), "{m0}"(m0v), "n"(NOP)
+                 : "memory");
 }
+template <int NOP = 4>
 __device__ __forceinline__ void lds_load4(__amdgpu_buffer_rsrc_t r, int voff, int soff, uint32_t m0v)
 {
-    asm volatile("buffer_load_dword %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff), "{m0}"(m0v) : "memory");
+    asm volatile("s_nop %4\n\tbuffer_load_dword %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff), "{m0}"(m0v), "n"(NOP)
+                 : "memory");
 }
+template <int NOP = 4>
 __device__ __forceinline__ void lds_load2(__amdgpu_buffer_rsrc_t r, int voff, int soff, uint32_t m0v)
 {
-    asm volatile("buffer_load_ushort %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff), "{m0}"(m0v) : "memory");
+    asm volatile("s_nop %4\n\tbuffer_load_ushort %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff), "{m0}"(m0v), "n"(NOP)
+                 : "memory");
 }
 template <int N>
 __device__ __forceinline__ void wait_vmcnt()

@@ -451,18 +451,18 @@ __global__ __launch_bounds__(256) void mfma_w4_pipe_kernel(PipeParams p)
         const int tc = min(t, last);
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-            lds_load16(ra, avo[q], tc * 64, lbase + OFF_A + st * A_ST + (wave * 64 + 16 * q) * 64);
+            lds_load16<0>(ra, avo[q], tc * 64, lbase + OFF_A + st * A_ST + (wave * 64 + 16 * q) * 64);
     };
     auto issue_b = [&](int g, int buf) {  // steps 4g .. 4g+3 -> buffer buf (CQ + 2 loads)
         const int gc = min(g, last >> 2);
 #pragma unroll
         for (int q = 0; q < CQ; ++q)
-            lds_load16(rb, cvo[q], gc * L::CROW, lbase + OFF_C + buf * CG + (wave * 64 + (64 / CQ) * q) * L::CROW);
-        lds_load16(rsc, svo, gc * 16, lbase + OFF_S + buf * SG + wave * 64 * 16);
+            lds_load16<0>(rb, cvo[q], gc * L::CROW, lbase + OFF_C + buf * CG + (wave * 64 + (64 / CQ) * q) * L::CROW);
+        lds_load16<0>(rsc, svo, gc * 16, lbase + OFF_S + buf * SG + wave * 64 * 16);
         if constexpr (B8)
-            lds_load4(rz, zvo, gc * 4, lbase + OFF_Z + buf * ZG + wave * 64 * 4);
+            lds_load4<0>(rz, zvo, gc * 4, lbase + OFF_Z + buf * ZG + wave * 64 * 4);
         else
-            lds_load2(rz, zvo, gc * 2, lbase + OFF_Z + buf * ZG + wave * 64 * 4);
+            lds_load2<0>(rz, zvo, gc * 2, lbase + OFF_Z + buf * ZG + wave * 64 * 4);
     };
     struct Raw {
         u32x4_t q[B8 ? 2 : 1];
@@ -561,7 +561,7 @@ __global__ __launch_bounds__(256) void mfma_w4_pipe_kernel(PipeParams p)
     // loads, so every wait below covers them too; rows past M read zero.
     {
         const int r = m0 + wave * 64 + lane;
-        lds_load4(buffer_rsrc(p.rexp, p.M * 4), r < p.M ? r * 4 : kPipeFar, 0, lbase + OFF_E + wave * 256);
+        lds_load4<0>(buffer_rsrc(p.rexp, p.M * 4), r < p.M ? r * 4 : kPipeFar, 0, lbase + OFF_E + wave * 256);
     }
     issue_b(0, 0);
     issue_b(1, 1);
