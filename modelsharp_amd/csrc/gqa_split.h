@@ -2,10 +2,11 @@
 // or 128) on the fp16 matrix cores at fp32-level accuracy.
 //
 // Every operand is held as two fp16 halves of its fp32 value, x = 2^e (xh + xl): 22 bits or
-// more, each product exact in the MFMA's fp32 sum, three products per operand pair
-// (xh yh + xh yl + xl yh, the dropped xl yl below 2^-22 of the product). That is 3 MFMAs of
-// 16 k against the fp32 unit's 4 of 4 k at the same issue cost per MFMA: 5.3 times the fp32
-// rate, with fewer rounded additions per sum.
+// more (a softmax weight: down to 2^-13 of the largest, and 2^-35 of that below), each product
+// exact in the MFMA's fp32 sum, three products per operand pair (xh yh + xh yl + xl yh, the
+// dropped xl yl below 2^-22 of the product). That is 3 MFMAs of 16 k against the fp32 unit's 4
+// of 4 k at the same issue cost per MFMA: 5.3 times the fp32 rate, with fewer rounded
+// additions per sum.
 //
 //   gqa_split_kv_kernel   one workgroup per 64-key chunk of K or of V: appends the new rows
 //                         to the present cache (as gqa_append_kernel does), and writes the
@@ -33,10 +34,10 @@
 // 2.7e-7 (4.5e-7). 32 / 8 heads of 96 over 1000 tokens: 60 us, 1111 before
 // (gqa_attention_kernel). The MFMAs are busy 31% of the time, the VALU (630 instructions per
 // wave and chunk) as much: what is left is the waits at each phase's barrier.
-// What the halves cannot carry (an infinity, a NaN, |q| or |k| >= 2^50, key or value rows
-// more than 2^12 apart in one scale: a row seen by queries that do not see the larger one
-// would lose its low bits) sends the query blocks that meet it to gqa_split_plain(), plain
-// fp32 arithmetic row by row.
+// What the halves cannot carry (an infinity, a NaN, |q| or |k| >= 2^50, key or value rows of a
+// chunk more than 2^12 apart: a row seen by queries that do not see the larger one would lose
+// its low bits; chunks of V more than 2^60 apart) sends the query blocks that meet it to
+// gqa_split_plain(), plain fp32 arithmetic row by row.
 #pragma once
 #include "gqa_args.h"
 #include "mfma_device.h"
@@ -46,11 +47,14 @@ namespace msnb {
 constexpr int kSplitChunk = 64;            // keys per chunk
 constexpr int kSplitSpecial = 0x7FFF;      // exponent of a chunk the halves cannot carry
 constexpr int kSplitEmpty = -1000;         // exponent of a row or chunk of zeros
-constexpr int kSplitSpread = 12;           // largest difference of row exponents under one scale
+constexpr int kSplitSpread = 12;           // largest difference of row exponents in a chunk
+constexpr int kSplitRange = 60;            // and of V's chunk exponents in a block's range
+constexpr int kSplitGrow = 4;              // the running maximum moves in steps above 2^4
+constexpr int kSplitWeight = 11;           // weights times 2^11 (or 2^10): at most 2^15 in fp16
 constexpr float kSplitMaxAbs = 1.125899906842624e15f;   // 2^50: scores stay finite in fp32
 
 // Workspace of a call: per (batch, kv head) `nch` chunks of [Kh | Kl | Vh | Vl], 128 D bytes
-// each, then the exponents [unit][nch][K, V largest, V smallest row, unused].
+// each, then the exponents [unit][nch][K, V, unused, unused].
 struct GqaSplitWs {
     uint8_t* img;
     int* exps;
@@ -211,15 +215,9 @@ __global__ __launch_bounds__(256) void gqa_split_kv_kernel(GqaArgs p, GqaSplitWs
             lo = min(lo, __shfl_xor(lo, o));
         }
         if (tid == 0) {
-            if (!is_v && hi != kSplitEmpty && hi - lo > kSplitSpread) hi = kSplitSpecial;
+            if (hi != kSplitEmpty && hi - lo > kSplitSpread) hi = kSplitSpecial;
             stat = hi;
-            int* const ex = w.exps + 4 * (int64_t)cid;
-            if (is_v) {
-                ex[1] = hi;
-                ex[2] = lo;
-            } else {
-                ex[0] = hi == kSplitEmpty ? 0 : hi;
-            }
+            w.exps[4 * (int64_t)cid + is_v] = !is_v && hi == kSplitEmpty ? 0 : hi;
         }
     }
     __syncthreads();
@@ -414,22 +412,21 @@ __global__ __launch_bounds__(128 * NW, 2) void gqa_split_kernel(GqaArgs p, GqaSp
     const int kmin = k_first(q0), kmax = k_last(min(q0 + BQ, p.Sq) - 1);
     const int ch0 = kmin / kSplitChunk, ch1 = kmax >= kmin ? kmax / kSplitChunk : ch0 - 1;
 
-    // V's common exponent over the range, and whether the halves carry every value
+    // whether the halves carry every value of the range
     const int4* const ex = reinterpret_cast<const int4*>(w.exps) + (int64_t)bg * w.nch;
     int ev_max = kSplitEmpty, ev_min = kSplitSpecial;
     for (int c = ch0 + lane; c <= ch1; c += 64) {
         const int4 e = ex[c];
         bad |= e.x == kSplitSpecial;
         ev_max = max(ev_max, e.y);
-        ev_min = min(ev_min, e.z);
+        if (e.y != kSplitEmpty) ev_min = min(ev_min, e.y);
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
         ev_max = max(ev_max, __shfl_xor(ev_max, o));
         ev_min = min(ev_min, __shfl_xor(ev_min, o));
     }
-    if (ev_max == kSplitEmpty) ev_max = 0;   // zeros only
-    else bad |= ev_max == kSplitSpecial || ev_max - ev_min > kSplitSpread;
+    bad |= ev_max == kSplitSpecial || (ev_max != kSplitEmpty && ev_max - ev_min > kSplitRange);
     if (__syncthreads_or(bad)) {
         gqa_split_plain<D, 2 * NW>(p, b, h, g, q0, min(q0 + BQ, p.Sq), reinterpret_cast<float*>(split_lds));
         return;
@@ -451,22 +448,39 @@ __global__ __launch_bounds__(128 * NW, 2) void gqa_split_kernel(GqaArgs p, GqaSp
 #pragma unroll
     for (int n = 0; n < NT; ++n) acc[n] = floatx16_t{};
     float m_run = -__builtin_inff(), l_run = 0.0f;   // base 2
+    int ev_run = kSplitEmpty;   // acc's exponent: V's of a chunk so far
     const float scale2 = p.scale * 1.44269504088896341f;   // scale * log2(e)
 
     // Phases of one group alternate S and P (below); group 1 starts one phase later, and the
     // group that would end first passes one more barrier, so that every wave passes as many.
     const int chunks = ch1 - ch0 + 1;
+    int4 ec = ex[max(min(ch0 + grp, ch1), 0)];
     if (ch0 + grp <= ch1) load(lk0, (ch0 + grp) * (4 * HALF));
     if (grp) lds_barrier();
     for (int ch = ch0 + grp; ch <= ch1; ch += 2) {
         const int c0 = ch * kSplitChunk;
-        const int ek = ex[ch].x, ev = ex[ch].y;
         wait_vmcnt<0>();   // this wave's part of K
+        // the chunk's exponents, loaded a chunk ahead: their use waits for every load before it,
+        // and here none is in flight
+        int ek = __builtin_amdgcn_readfirstlane(ec.x), ev = __builtin_amdgcn_readfirstlane(ec.y);
+        asm volatile("" : "+s"(ek), "+s"(ev));
+        ec = ex[min(ch + 2, ch1)];
         lds_barrier();     // the group's; and the previous chunk's V readers are done
         load(lv0, ch * (4 * HALF) + 2 * HALF);
         const bool live = c0 <= wlast && c0 + kSplitChunk > wfirst;
         half8_t ph[4], pl[4];
         if (live) {
+            // The sums follow V's exponent from chunk to chunk (exactly: powers of two, at most
+            // 2^60), except by 1 down, which the weights take: so a weight of 1 is 2^10 or 2^11
+            // in fp16, and one of 2^-13 still has 22 bits.
+            if (ev > ev_run || (ev < ev_run - 1 && ev != kSplitEmpty)) {   // uniform
+                const float move = __builtin_amdgcn_ldexpf(1.0f, ev_run - ev);
+                ev_run = ev;
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) acc[n][v] = acc[n][v] * move;
+            }
             // S^T: two tiles of 32 keys; the small cross products have sums of their own, so
             // that they do not add to the roundings of the main one
             floatx16_t st[2];
@@ -503,15 +517,13 @@ __global__ __launch_bounds__(128 * NW, 2) void gqa_split_kernel(GqaArgs p, GqaSp
             cm = fmaxf(cm, xor32_value(cm));
             // score = st * f; f > 0 (the host sends other scales elsewhere) and not denormal
             const float f = fmaxf(__builtin_amdgcn_ldexpf(scale2, eq + ek), 7.5e-37f);
-            // The maximum moves only when it grows by more than 2^8, so that the sums are seldom
-            // rescaled; weights then reach 2^8.
-            const float m_new = cm * f > m_run + 8.0f ? cm * f : m_run;
+            // The maximum moves only when it grows by more than 2^4, so that the sums are seldom
+            // rescaled; weights then reach 2^4.
+            const float m_new = cm * f > m_run + (float)kSplitGrow ? cm * f : m_run;
             const bool none = m_new == -__builtin_inff();   // no key of this query so far
             const float alpha = none ? 1.0f : __builtin_amdgcn_exp2f(m_run - m_new);
             const float msub = none ? 0.0f : m_new;   // masked scores are -inf: weight 0 either way
-            // weights times 2^7 (at most 2^15 in fp16, room below 1) and V's chunk exponent over the
-            // common one
-            const float gv = __builtin_amdgcn_ldexpf(128.0f, max(ev - ev_max, -200));
+            const float gv = (float)(ev == ev_run ? 1 << kSplitWeight : 1 << (kSplitWeight - 1));
             float ls = 0.0f;
 #pragma unroll
             for (int s = 0; s < 4; ++s)
@@ -559,10 +571,11 @@ __global__ __launch_bounds__(128 * NW, 2) void gqa_split_kernel(GqaArgs p, GqaSp
     if (grp) {
         xs[0] = m_run;
         xs[XS] = l_run;
+        xs[2 * XS] = (float)ev_run;
 #pragma unroll
         for (int n = 0; n < NT; ++n)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) xs[(2 + 16 * n + v) * XS] = acc[n][v];
+            for (int v = 0; v < 16; ++v) xs[(3 + 16 * n + v) * XS] = acc[n][v];
     }
     lds_barrier();
     if (grp) return;
@@ -571,12 +584,15 @@ __global__ __launch_bounds__(128 * NW, 2) void gqa_split_kernel(GqaArgs p, GqaSp
         const float f0 = m_run == m ? 1.0f : __builtin_amdgcn_exp2f(m_run - m);   // also for no keys at all
         const float f1 = m1 == m ? 1.0f : __builtin_amdgcn_exp2f(m1 - m);
         l_run = l_run * f0 + xs[XS] * f1;
+        const int ev1 = (int)xs[2 * XS], ev = max(ev_run, ev1);
+        const float g0 = __builtin_amdgcn_ldexpf(f0, ev_run - ev), g1 = __builtin_amdgcn_ldexpf(f1, ev1 - ev);
+        ev_run = ev;
 #pragma unroll
         for (int n = 0; n < NT; ++n)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[n][v] = acc[n][v] * f0 + xs[(2 + 16 * n + v) * XS] * f1;
+            for (int v = 0; v < 16; ++v) acc[n][v] = acc[n][v] * g0 + xs[(3 + 16 * n + v) * XS] * g1;
     }
-    // acc[n][v] is O[query][channel 32 n + 8 (v / 4) + 4 hf + v % 4] * l * 2^(7 - ev_max)
+    // acc[n][v] is O[query][channel 32 n + 8 (v / 4) + 4 hf + v % 4] * l * 2^(kSplitWeight - ev_run)
     if (q_in) {
         const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
         float* orow = p.out + (int64_t)(b * p.Sq + qi) * p.H * D + h * D + 4 * hf;
@@ -584,7 +600,7 @@ __global__ __launch_bounds__(128 * NW, 2) void gqa_split_kernel(GqaArgs p, GqaSp
         for (int n = 0; n < NT; ++n)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                auto o = [&](int i) { return __builtin_amdgcn_ldexpf(acc[n][4 * j + i] * inv, ev_max - 7); };
+                auto o = [&](int i) { return __builtin_amdgcn_ldexpf(acc[n][4 * j + i] * inv, ev_run - kSplitWeight); };
                 *reinterpret_cast<float4*>(orow + 32 * n + 8 * j) = float4{o(0), o(1), o(2), o(3)};
             }
     }

@@ -304,7 +304,7 @@ def test_skipnorm_rejects_outputs_over_inputs(gpu):
 
 
 # ---- GroupQueryAttention ---------------------------------------------------------------------
-from test_oracle_decoder import GQA_CASES, make_case   # noqa: E402
+from test_oracle_decoder import GQA_CASES, gqa_f64, make_case   # noqa: E402
 
 
 def run_device_gqa(d, q, k, v, pk, pv, sl, cos, sin, capacity=None, workspace=False):
@@ -436,6 +436,22 @@ def test_gqa_split_extreme_values(gpu, where, value):
         rows = np.abs(np.where(ok, ref, 0.0)).reshape(150 * 4, 128).max(axis=1, keepdims=True)
         err = np.abs(np.where(ok, out - ref, 0.0)).reshape(150 * 4, 128)
     assert np.all(err <= 1e-5 * rows)
+
+
+@pytest.mark.parametrize("exps", [(-11, 0, 0, 0), (0, -11, 0, -11), (-20, 0, -30, 20), (10, 0, -10, -25)], ids=str)
+@pytest.mark.parametrize("D", [64, 96, 128])
+def test_gqa_split_values_of_different_magnitude(gpu, D, exps):
+    """64-key stretches of V whose magnitudes differ by powers of two: every output row, those of
+    the queries that see the small stretches alone among them, is as close to 64 bits as two
+    fp16 halves are: 2^-22 each for the weight, for V and for the dropped product of low halves
+    (in 2-norm over the row, fp32 sums included; measured 2e-7 or less)."""
+    d, q, k, v, *_ = make_case(233, B=1, Sq=256, H=4, KH=2, D=D, past=0, rotary=False, cos_rows=8)
+    v *= np.exp2(np.repeat(np.asarray(exps, dtype=np.float32), 64))[None, :, None]
+    out, _, _ = run_device_gqa(d, q, k, v, None, None, None, None, None, workspace=True)
+    ref = np.asarray(gqa_f64(d, q, k, v, None, None, None, None, None)[0]).reshape(-1, D)
+    err = np.linalg.norm(out.reshape(-1, D) - ref, axis=-1) / np.linalg.norm(ref, axis=-1)
+    log(f"split D={D} V exponents {exps}: largest row error {err.max():.2e}")
+    assert err.max() <= 3 * 2.0 ** -22
 
 
 @pytest.mark.parametrize("workspace", [False, True], ids=["one_split", "key_splits"])
