@@ -37,7 +37,7 @@
 // What the halves cannot carry (an infinity, a NaN, |q| or |k| >= 2^50, key or value rows of a
 // chunk more than 2^12 apart: a row seen by queries that do not see the larger one would lose
 // its low bits; chunks of V more than 2^60 apart) sends the query blocks that meet it to
-// gqa_split_plain(), plain fp32 arithmetic row by row.
+// gqa_split_f32(), the same tiles in fp32.
 #pragma once
 #include "gqa_args.h"
 #include "mfma_device.h"
@@ -233,58 +233,178 @@ __global__ __launch_bounds__(256) void gqa_split_kv_kernel(GqaArgs p, GqaSplitWs
     }
 }
 
-// Queries [q0, qend) of (b, h) in plain fp32, one after another (scores as gqa_rows_kernel
-// forms them: the maximum first, then the weights; only visible keys are touched).
-template <int D, int NW>
-__device__ void gqa_split_plain(const GqaArgs& p, int b, int h, int g, int q0, int qend, float* lds)
+// The wave's 32 query rows [qw0, qw0 + 32), rotated, to its part of LDS: 16-byte chunk c of row
+// r at chunk (c + r) % (D / 4). They come in whole (a lane per row would touch 32 lines per load).
+typedef __attribute__((address_space(3))) floatx4_t lds_f4_t;
+typedef __attribute__((address_space(3))) float lds_f_t;
+template <int D, int UNROLL>
+__device__ __forceinline__ void gqa_split_stage_q(const GqaArgs& p, lds_f4_t* xq, int b, int h, int qw0, int lane)
 {
-    constexpr int NT = 64 * NW, R = (D + NT - 1) / NT;
-    float* const qs = lds;   // NW: all waves of the workgroup
-    float* const ps = lds + D;
-    float* const red = ps + NT;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    int bound = p.total - 1;
-    if (p.seqlens_len > 0) bound = min(bound, p.seqlens[min(b, p.seqlens_len - 1)]);
-    const float* const kb = p.pk + (int64_t)(b * p.kvH + g) * p.cap * D;
-    const float* const vb = p.pv + (int64_t)(b * p.kvH + g) * p.cap * D;
-    for (int qi = q0; qi < qend; ++qi) {
-        const int q_abs = p.past + qi, last = min(q_abs, bound);
-        const int first = p.window >= 0 ? max(0, q_abs - p.window + 1) : 0;
-        const float* qrow = p.q + (int64_t)(b * p.Sq + qi) * p.q_stride + h * D;
-        const int pos = rotary_pos(q_abs, p);
-        __syncthreads();
-        for (int d = tid; d < D; d += NT) qs[d] = rotated(qrow, d, pos, p);
-        __syncthreads();
-        auto score = [&](int key) {
-            float s = 0.0f;
-            for (int d = 0; d < D; ++d) s = __builtin_fmaf(qs[d], kb[(int64_t)key * D + d], s);
-            return s * p.scale;
-        };
-        float mx = -__builtin_inff();
-        for (int key = first + tid; key <= last; key += NT) mx = fmaxf(mx, score(key));
-        for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-        if (lane == 0) red[wave] = mx;
-        __syncthreads();
-        for (int w = 0; w < NW; ++w) mx = fmaxf(mx, red[w]);
-        float acc[R], sum = 0.0f;
-        for (int r = 0; r < R; ++r) acc[r] = 0.0f;
-        for (int base = first; base <= last; base += NT) {
-            const int n = min(NT, last + 1 - base);
-            __syncthreads();
-            if (tid < n) ps[tid] = expf(score(base + tid) - mx);
-            __syncthreads();
-            for (int j = 0; j < n; ++j) {
-                sum = sum + ps[j];
-                for (int r = 0; r < R; ++r)
-                    if (tid + r * NT < D)
-                        acc[r] = __builtin_fmaf(ps[j], vb[(int64_t)(base + j) * D + tid + r * NT], acc[r]);
+    constexpr int CH = D / 4, ITS = 32 * CH / 64;
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll UNROLL
+    for (int i = 0; i < ITS; ++i) {
+        const int u = lane + 64 * i, r = u / CH, c = u - r * CH, row = min(qw0 + r, p.Sq - 1);
+        xq[r * CH + (c + r) % CH] = rotated4<D>(p.q + (int64_t)(b * p.Sq + row) * p.q_stride + h * D, 4 * c,
+                                                rotary_pos(p.past + row, p), p);
+    }
+    __builtin_amdgcn_wave_barrier();
+}
+
+// A query block that the halves cannot carry, in fp32 on the matrix cores: the same tiles and
+// work split, K, V and the staged queries read as they are. Two passes over the keys: the
+// maximum of every score first, then the weights against it, so that no sum is larger than the
+// plain definition's. Infinities and NaN of rows that a query does not see do not reach it:
+// scores are masked, and chunks of V that hold such values and that not all queries see whole
+// are added key by key. `lds` holds the queries (gqa_split_stage_q); every wave of the
+// workgroup is here, and ends here (so that the halves need no registers of its). 2048 tokens
+// of 28 / 4 heads of 128, every block: 0.6 ms (41 ms row by row, one query after another).
+template <int D, int NW>
+__device__ __forceinline__ void gqa_split_f32(const GqaArgs& p, const int4* ex, lds_f4_t* lds, int bg, int b, int h,
+                                              int qw0, int wave2, int lane, int ch0, int ch1, int wfirst, int wlast,
+                                              int kf_q, int kl_q)
+{
+    constexpr int T = D / 16, NT = D / 32, CH = D / 4;
+    const int l32 = lane & 31, hf = lane >> 5, grp = wave2 / NW, wave = wave2 % NW;
+    lds_f4_t* const xq = lds + wave2 * 32 * CH;
+    const int total = p.total;
+    // the unit's rows: loads past the last read zero
+    const int64_t unit = (int64_t)bg * p.cap * D;
+    const __amdgpu_buffer_rsrc_t rk = buffer_rsrc(p.pk + unit, total * D * 4);
+    const __amdgpu_buffer_rsrc_t rv = buffer_rsrc(p.pv + unit, total * D * 4);
+    const float scale2 = p.scale * 1.44269504088896341f;
+    auto live = [&](int c0) { return c0 <= wlast && c0 + kSplitChunk > wfirst; };
+    auto key_of = [&](int c0, int kt, int v) { return c0 + 32 * kt + 8 * (v >> 2) + 4 * hf + (v & 3); };
+    auto scores = [&](int c0, floatx16_t (&st)[2]) {   // base 2, masked
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) {
+            st[kt] = floatx16_t{};
+            const int kr = ((c0 + l32) * D + 8 * hf) * 4;
+#pragma unroll 2
+            for (int t = 0; t < T; ++t) {
+                floatx4_t a[2], x[2];
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    a[e] = __builtin_bit_cast(floatx4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                             rk, kr, (32 * kt * D + 16 * t + 4 * e) * 4, 0));
+                    x[e] = xq[l32 * CH + (4 * t + 2 * hf + e + l32) % CH];
+                }
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    st[kt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i >> 2][i & 3], x[i >> 2][i & 3], st[kt], 0, 0, 0);
+            }
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int key = key_of(c0, kt, v);
+                st[kt][v] = key >= kf_q && key <= kl_q ? st[kt][v] * scale2 : -__builtin_inff();
             }
         }
-        const float inv = sum > 0.0f ? 1.0f / sum : sum == 0.0f ? 0.0f : sum;   // a NaN sum stays one
-        for (int r = 0; r < R; ++r)
-            if (tid + r * NT < D)
-                p.out[(int64_t)(b * p.Sq + qi) * p.H * D + h * D + tid + r * NT] = last >= first ? acc[r] * inv : 0.0f;
+    };
+
+    float mx = -__builtin_inff();
+    for (int ch = ch0 + grp; ch <= ch1; ch += 2) {
+        const int c0 = ch * kSplitChunk;
+        if (!live(c0)) continue;
+        floatx16_t st[2];
+        scores(c0, st);
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) mx = fmaxf(mx, st[kt][v]);
     }
+    mx = fmaxf(mx, xor32_value(mx));
+    lds_f_t* const ms = (lds_f_t*)lds;   // both groups' maxima, over the queries
+    __syncthreads();
+    ms[wave2 * 64 + lane] = mx;
+    __syncthreads();
+    mx = fmaxf(ms[wave * 64 + lane], ms[(NW + wave) * 64 + lane]);
+    __syncthreads();
+    gqa_split_stage_q<D, 1>(p, xq, b, h, qw0, lane);
+    floatx16_t acc[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[n] = floatx16_t{};
+    // every visible score -inf: weights e^(-inf + inf), as the definition has them
+    float l_run = mx == -__builtin_inff() && kl_q >= kf_q ? __builtin_nanf("") : 0.0f;
+    const float msub = mx == -__builtin_inff() ? 0.0f : mx;
+    for (int ch = ch0 + grp; ch <= ch1; ch += 2) {
+        const int c0 = ch * kSplitChunk;
+        if (!live(c0)) continue;
+        floatx16_t st[2];
+        scores(c0, st);
+        float ls = 0.0f;
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                st[kt][v] = exp2f(st[kt][v] - msub);
+                ls = ls + st[kt][v];
+            }
+        l_run = l_run + ls + xor32_value(ls);
+        if (ex[ch].y != kSplitSpecial || __all(c0 >= kf_q && c0 + kSplitChunk - 1 <= kl_q)) {
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) {
+                        const float y = __builtin_bit_cast(
+                            float, __builtin_amdgcn_raw_buffer_load_b32(
+                                       rv, ((c0 + 4 * hf) * D + l32) * 4, ((32 * kt + 8 * (v >> 2) + (v & 3)) * D + 32 * n) * 4, 0));
+                        acc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(y, st[kt][v], acc[n], 0, 0, 0);
+                    }
+                    if ((v & 3) == 3) __builtin_amdgcn_sched_barrier(0);   // four keys' loads in flight, not 32
+                }
+        } else {   // the weights [key][query] over the wave's queries, which come back afterwards
+            lds_f_t* const ps = (lds_f_t*)xq;
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) ps[(key_of(c0, kt, v) - c0) * 32 + l32] = st[kt][v];
+            __builtin_amdgcn_wave_barrier();
+            for (int k = 0; k < kSplitChunk && c0 + k < total; ++k) {
+                const float w = ps[k * 32 + l32];
+                const bool seen = c0 + k >= kf_q && c0 + k <= kl_q;
+#pragma unroll
+                for (int n = 0; n < NT; ++n) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const auto y = __builtin_bit_cast(floatx4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                                         rv, ((c0 + k) * D + 4 * hf) * 4, (32 * n + 8 * j) * 4, 0));
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            acc[n][4 * j + i] = seen ? __builtin_fmaf(w, y[i], acc[n][4 * j + i]) : acc[n][4 * j + i];
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            gqa_split_stage_q<D, 1>(p, xq, b, h, qw0, lane);
+        }
+    }
+    // group 1's sums to group 0, through LDS
+    constexpr int XS = 64 * NW;
+    lds_f_t* const xs = ms + wave * 64 + lane;
+    __syncthreads();
+    if (grp) {
+        xs[0] = l_run;
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) xs[(1 + 16 * n + v) * XS] = acc[n][v];
+    }
+    __syncthreads();
+    const int qi = qw0 + l32;
+    if (grp || qi >= p.Sq) return;
+    l_run = l_run + xs[0];
+    const float inv = l_run > 0.0f ? 1.0f / l_run : l_run == 0.0f ? 0.0f : l_run;   // a NaN sum stays one
+    float* const orow = p.out + (int64_t)(b * p.Sq + qi) * p.H * D + h * D + 4 * hf;
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            auto o = [&](int i) { return (acc[n][4 * j + i] + xs[(1 + 16 * n + 4 * j + i) * XS]) * inv; };
+            *reinterpret_cast<f4u_t*>(orow + 32 * n + 8 * j) = f4u_t{o(0), o(1), o(2), o(3)};
+        }
 }
 
 // Work items: (query block, head), the latest (heaviest) blocks first. The workgroups of one
@@ -368,23 +488,16 @@ __global__ __launch_bounds__(128 * NW, 2) void gqa_split_kernel(GqaArgs p, GqaSp
     auto k_last = [&](int qi) { return min(p.past + qi, bound); };
 
     // this lane's query: B operand of k-step t, channels 16 t + 8 hf + [0, 8). The wave's 32
-    // rows come in whole (a lane per row would touch 32 lines per load) and cross over in
-    // its part of LDS, 16-byte chunk c of row r at chunk (c + r) % (D / 4).
+    // rows cross over in its part of LDS.
     const int qw0 = q0 + 32 * wave, qi = qw0 + l32;
     const bool q_in = qi < p.Sq;
     half8_t qh[T], ql[T];
     int eq;
     bool bad = false;
     {
-        constexpr int CH = D / 4, ITS = 32 * CH / 64;
-        floatx4_t* const xq = reinterpret_cast<floatx4_t*>(split_lds) + wave2 * 32 * CH;
-#pragma unroll 4
-        for (int i = 0; i < ITS; ++i) {
-            const int u = lane + 64 * i, r = u / CH, c = u - r * CH, row = min(qw0 + r, p.Sq - 1);
-            xq[r * CH + (c + r) % CH] = rotated4<D>(p.q + (int64_t)(b * p.Sq + row) * p.q_stride + h * D, 4 * c,
-                                                    rotary_pos(p.past + row, p), p);
-        }
-        __builtin_amdgcn_wave_barrier();
+        constexpr int CH = D / 4;
+        lds_f4_t* const xq = (lds_f4_t*)split_lds + wave2 * 32 * CH;
+        gqa_split_stage_q<D, 4>(p, xq, b, h, qw0, lane);
         float x[T][8], mx = 0.0f;
 #pragma unroll
         for (int t = 0; t < T; ++t) {
@@ -427,9 +540,9 @@ __global__ __launch_bounds__(128 * NW, 2) void gqa_split_kernel(GqaArgs p, GqaSp
         ev_min = min(ev_min, __shfl_xor(ev_min, o));
     }
     bad |= ev_max == kSplitSpecial || (ev_max != kSplitEmpty && ev_max - ev_min > kSplitRange);
-    if (__syncthreads_or(bad)) {
-        gqa_split_plain<D, 2 * NW>(p, b, h, g, q0, min(q0 + BQ, p.Sq), reinterpret_cast<float*>(split_lds));
-        return;
+    if (__builtin_amdgcn_readfirstlane(__syncthreads_or(bad))) {
+        gqa_split_f32<D, NW>(p, ex, (lds_f4_t*)split_lds, bg, b, h, qw0, wave2, lane, ch0, ch1, wfirst, wlast, kf_q, kl_q);
+        __builtin_amdgcn_endpgm();
     }
 
     // chunk images -> LDS: wave w moves every NW-th KB
@@ -601,7 +714,7 @@ __global__ __launch_bounds__(128 * NW, 2) void gqa_split_kernel(GqaArgs p, GqaSp
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 auto o = [&](int i) { return __builtin_amdgcn_ldexpf(acc[n][4 * j + i] * inv, ev_run - kSplitWeight); };
-                *reinterpret_cast<float4*>(orow + 32 * n + 8 * j) = float4{o(0), o(1), o(2), o(3)};
+                *reinterpret_cast<f4u_t*>(orow + 32 * n + 8 * j) = f4u_t{o(0), o(1), o(2), o(3)};
             }
     }
 }

@@ -454,6 +454,81 @@ def test_gqa_split_values_of_different_magnitude(gpu, D, exps):
     assert err.max() <= 3 * 2.0 ** -22
 
 
+# Query blocks that the halves cannot carry (gqa_split_f32), every head_dim (64 from 192 keys on), both workgroup sizes
+# (128 queries from 256 workgroups on), ragged last blocks and chunks, a cached past, lengths
+# and windows that end inside a chunk with a special value.
+SPLIT_F32_CASES = [
+    dict(B=1, Sq=200, H=4, KH=2, past=0, cos_rows=200),
+    dict(B=1, Sq=129, H=128, KH=8, past=65, cos_rows=200),
+    dict(B=2, Sq=161, H=64, KH=4, past=40, seqlens=[95, 190], cos_rows=201),
+    dict(B=1, Sq=140, H=6, KH=3, past=70, window=90, packed=True, cos_rows=210),
+    dict(B=3, Sq=270, H=2, KH=1, past=0, window=150, interleaved=True, cos_rows=270),
+]
+
+
+@pytest.mark.parametrize("what", ["v_spread", "v_inf", "v_nan", "k_nan", "k_spread", "k_inf", "q_huge"])
+@pytest.mark.parametrize("case", SPLIT_F32_CASES, ids=lambda c: f"H{c['H']}_past{c['past']}_B{c['B']}")
+@pytest.mark.parametrize("D", [64, 96, 128])
+def test_gqa_split_f32_blocks(gpu, D, case, what):
+    d, q, k, v, pk, pv, sl, cos, sin = make_case(seed=241, D=D, **case)
+    packed, qh, kh = case.get("packed"), d.num_heads * D, d.kv_num_heads * D
+    kk, vv = (q[..., qh:qh + kh], q[..., qh + kh:]) if packed else (k, v)
+    rows = [20, 100]   # new rows; with a past they lie in the second and third chunk
+    value = {"spread": 2.0 ** 14, "inf": np.inf, "nan": np.nan, "huge": 2e15}[what.split("_")[1]]
+    for r in rows:
+        if what == "q_huge":
+            q[0, r, 5] = value
+        elif what.endswith("spread"):
+            (vv if what[0] == "v" else kk)[0, r, :D] *= np.float32(value)
+        else:
+            (vv if what[0] == "v" else kk)[0, r, 5] = value
+    with np.errstate(all="ignore"):
+        ref, rk, rv = oracle.gqa(d, q, k, v, pk, pv, sl, cos, sin)
+        out, PK, PV = run_device_gqa(d, q, k, v, pk, pv, sl, cos, sin, capacity=d.past_seq + d.kv_seq + 3, workspace=True)
+        assert np.array_equal(PK, rk, equal_nan=True) and np.array_equal(PV, rv, equal_nan=True)
+        assert np.array_equal(np.isnan(out), np.isnan(ref)) and np.array_equal(np.isinf(out), np.isinf(ref))
+        ok = np.isfinite(ref)
+        rowmax = np.abs(np.where(ok, ref, 0.0)).reshape(-1, D).max(axis=1, keepdims=True)
+        err = np.abs(np.where(ok, out - ref, 0.0)).reshape(-1, D)
+    # a score of 2^14 times the usual size (5e4) is rounded by 3e-3 in fp32, which is its
+    # weight's relative error: a few of them on either side
+    bar = 1e-5 if what not in ("k_spread", "q_huge") else 2e-2
+    worst = float(np.max(err / np.maximum(rowmax, 1e-30)))
+    log(f"split f32 D={D} {what} {case}: {worst:.2e}")
+    assert worst <= bar
+
+
+def test_gqa_split_f32_time(gpu):
+    """A prompt whose values the halves cannot carry costs a few times the ordinary one, not
+    hundreds (the definition's row by row arithmetic took tens of milliseconds)."""
+    import torch
+    H, KH, D, S = 28, 4, 128, 2048
+    d = native.GqaDesc(batch=1, q_seq=S, kv_seq=S, num_heads=H, kv_num_heads=KH, head_dim=D, present_capacity=S,
+                       local_window_size=-1)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    q, k, v = (torch.randn((1, S, n * D), device="cuda", generator=g) for n in (H, KH, KH))
+    out, PK, PV = torch.empty_like(q), *(torch.empty((1, KH, S, D), device="cuda") for _ in range(2))
+    ws = torch.empty(native.gqa_workspace_size(d) // 4, device="cuda")
+
+    def run(vals):
+        t = []
+        for _ in range(4):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            native.gqa(d, q.data_ptr(), k.data_ptr(), vals.data_ptr(), None, None, None, None, None, out.data_ptr(),
+                       PK.data_ptr(), PV.data_ptr(), ws.data_ptr(), ws.numel() * 4, torch.cuda.current_stream().cuda_stream)
+            b.record()
+            torch.cuda.synchronize()
+            t.append(a.elapsed_time(b))
+        return min(t)
+
+    spread = v.clone()
+    spread[0, 3] *= 2.0 ** 14
+    plain, special = run(v), run(spread)
+    log(f"prompt attention: {plain * 1e3:.0f} us, in fp32 {special * 1e3:.0f} us")
+    assert special <= 20 * plain
+
+
 @pytest.mark.parametrize("workspace", [False, True], ids=["one_split", "key_splits"])
 @pytest.mark.parametrize("Sq,past,KH", [(1, 2047, 8), (1, 4095, 32), (128, 0, 8), (16, 300, 8)])
 def test_gqa_7b_shapes(gpu, Sq, past, KH, workspace):
