@@ -692,3 +692,26 @@ def test_block_gemm_beyond_the_allocation_free_scratch(gpu):
         np.max(np.abs(a[rows]), axis=1, keepdims=True).astype(np.float64) * np.abs(W).sum(axis=1)[None, :])
     assert_within(y.cpu().numpy()[rows], ref, allowed, "beyond the scratch")
     w.close()
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M", [1, 5, 16])
+def test_chunk_gemv_at_the_top_of_fp32(gpu, M, bits):
+    """Activations whose products with the codes pass the range of fp32, while those with the
+    scaled weights stay far inside it; one row of ordinary activations among them, and rows of
+    infinities and NaN, whose outputs are the oracle's."""
+    op = Op("chunk_top", 96, 37, 32, True, bits=bits)
+    b, s, _ = workloads.make_weights(op, seed=bits + M)
+    zpf = float_zero_points(op, seed=M)
+    a = workloads.make_activations(M, op.K, seed=M)
+    top = 3e37 if bits == 4 else 2e36   # times 32 or 16 codes up to 15 or 255, and times 0.01 of that
+    a[:(M + 1) // 2] = np.sign(a[:(M + 1) // 2]) * np.float32(top)
+    w = native.NBitsWeights(b, s, zpf, op.N, op.K, op.bits, op.block_size)
+    kernel, _ = check_against_oracle(w, a, b, s, None, zpf, op, f"chunk bits={bits} M={M} at {top}")
+    assert kernel == "gemv_general"
+    a[0, 3], a[-1, 7] = np.inf, np.nan
+    with np.errstate(all="ignore"):
+        ref = oracle.matmul_nbits(a, b, s, None, op.N, op.K, op.bits, op.block_size, zp_float=zpf)
+    y = w.gemm(a)
+    assert np.array_equal(np.isnan(y), np.isnan(ref)) and np.array_equal(np.isinf(y), np.isinf(ref))
+    w.close()
