@@ -313,6 +313,7 @@ __device__ __forceinline__ void gqa_split_f32(const GqaArgs& p, const int4* ex, 
             for (int v = 0; v < 16; ++v) mx = fmaxf(mx, st[kt][v]);
     }
     mx = fmaxf(mx, xor32_value(mx));
+    lds_f_t* const ps = (lds_f_t*)xq;
     lds_f_t* const ms = (lds_f_t*)lds;   // both groups' maxima, over the queries
     __syncthreads();
     ms[wave2 * 64 + lane] = mx;
@@ -340,28 +341,25 @@ __device__ __forceinline__ void gqa_split_f32(const GqaArgs& p, const int4* ex, 
                 ls = ls + st[kt][v];
             }
         l_run = l_run + ls + xor32_value(ls);
+        // the weights [key][query] over the wave's queries, which come back afterwards
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) ps[(key_of(c0, kt, v) - c0) * 32 + l32] = st[kt][v];
+        __builtin_amdgcn_wave_barrier();
         if (ex[ch].y != kSplitSpecial || __all(c0 >= kf_q && c0 + kSplitChunk - 1 <= kl_q)) {
+#pragma unroll 4
+            for (int k = 0; k < kSplitChunk; k += 2) {
+                const float w = ps[(k + hf) * 32 + l32];
 #pragma unroll
-            for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-#pragma unroll
-                    for (int n = 0; n < NT; ++n) {
-                        const float y = __builtin_bit_cast(
-                            float, __builtin_amdgcn_raw_buffer_load_b32(
-                                       rv, ((c0 + 4 * hf) * D + l32) * 4, ((32 * kt + 8 * (v >> 2) + (v & 3)) * D + 32 * n) * 4, 0));
-                        acc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(y, st[kt][v], acc[n], 0, 0, 0);
-                    }
-                    if ((v & 3) == 3) __builtin_amdgcn_sched_barrier(0);   // four keys' loads in flight, not 32
+                for (int n = 0; n < NT; ++n) {
+                    const float y = __builtin_bit_cast(
+                        float, __builtin_amdgcn_raw_buffer_load_b32(rv, ((c0 + k + hf) * D + l32) * 4, 128 * n, 0));
+                    acc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(y, w, acc[n], 0, 0, 0);
                 }
-        } else {   // the weights [key][query] over the wave's queries, which come back afterwards
-            lds_f_t* const ps = (lds_f_t*)xq;
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) ps[(key_of(c0, kt, v) - c0) * 32 + l32] = st[kt][v];
-            __builtin_amdgcn_wave_barrier();
+            }
+        } else {
             for (int k = 0; k < kSplitChunk && c0 + k < total; ++k) {
                 const float w = ps[k * 32 + l32];
                 const bool seen = c0 + k >= kf_q && c0 + k <= kl_q;
@@ -378,8 +376,8 @@ __device__ __forceinline__ void gqa_split_f32(const GqaArgs& p, const int4* ex, 
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
-            gqa_split_stage_q<D, 1>(p, xq, b, h, qw0, lane);
         }
+        gqa_split_stage_q<D, 1>(p, xq, b, h, qw0, lane);
     }
     // group 1's sums to group 0, through LDS
     constexpr int XS = 64 * NW;
@@ -552,7 +550,8 @@ __global__ __launch_bounds__(128 * NW, 2) void gqa_split_kernel(GqaArgs p, GqaSp
 #pragma unroll
         for (int i = 0; i < 2 * HALF / 1024 / NW; ++i) {
             const int o = (i * NW + wave) * 1024;
-            lds_load16(rimg, 16 * lane, src + o, dst + o);
+            if (i == 0) lds_load16(rimg, 16 * lane, src + o, dst + o);
+            else lds_load16<0>(rimg, 16 * lane, src + o, dst + o);   // the resource is in place
         }
     };
     static_assert(2 * HALF % (1024 * NW) == 0, "a chunk's halves divide over the waves");
