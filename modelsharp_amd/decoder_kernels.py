@@ -542,7 +542,7 @@ class HipGroupQueryAttentionKernel(IKernel):
     def __init__(self):
         self._dev = _DeviceInputs()
         self._caches: dict[str, _Cache] = {}
-        self._workspace: dict[str, object] = {}   # key-split workspace per node (ms_hip_gqa_workspace_size)
+        self._workspace: dict[str, object] = {}   # a decode step's key-split workspace per node
 
     def _cache_for(self, node, B, KH, D, past_k, past_v, past, total, device):
         torch = _torch()
@@ -562,6 +562,24 @@ class HipGroupQueryAttentionKernel(IKernel):
         c = _Cache(k, v, cap)
         self._caches[node.name] = c
         return c, False
+
+    def _workspace_for(self, node, q_seq, ws_bytes, device):
+        """The call's workspace, or None (the library then takes a kernel that needs none). A
+        decode step's is small and kept per node. A prompt's is as large as its keys and values:
+        it comes from torch's allocator for this call alone, so that the layers of a model share
+        one and nothing of it stays through decode."""
+        torch = _torch()
+        if not ws_bytes:
+            return None
+        ws = self._workspace.get(node.name) if q_seq <= 8 else None
+        if ws is None or ws.numel() * 4 < ws_bytes:
+            try:
+                ws = torch.empty((ws_bytes + 3) // 4, dtype=torch.float32, device=device)
+            except torch.OutOfMemoryError:
+                return None
+            if q_seq <= 8:
+                self._workspace[node.name] = ws
+        return ws
 
     def execute(self, node: GraphNode, ctx: GraphContext) -> None:
         torch = _torch()
@@ -646,13 +664,8 @@ class HipGroupQueryAttentionKernel(IKernel):
                            scale=_attr_float(node, "scale", 0.0),
                            seqlens_len=0 if seqlens is None else int(seqlens.numel()))
         out = torch.empty((B, Sq, H * D), dtype=torch.float32, device=q.device)
-        ws_bytes = native.gqa_workspace_size(d)
-        ws = None
-        if ws_bytes:
-            ws = self._workspace.get(node.name)
-            if ws is None or ws.numel() * 4 < ws_bytes:
-                ws = torch.empty((ws_bytes + 3) // 4, dtype=torch.float32, device=q.device)
-                self._workspace[node.name] = ws
+        ws = self._workspace_for(node, Sq, native.gqa_workspace_size(d), q.device)
+        ws_bytes = 0 if ws is None else ws.numel() * 4
         ptr = lambda t: None if t is None else t.data_ptr()   # noqa: E731
         native.gqa(d, q.data_ptr(), ptr(k), ptr(v), ptr(pk_src), ptr(pv_src), ptr(seqlens), ptr(cos), ptr(sin),
                    out.data_ptr(), cache.k.data_ptr(), cache.v.data_ptr(), ptr(ws), ws_bytes, _stream(q))

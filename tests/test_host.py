@@ -535,3 +535,25 @@ def test_engine_marks_initializers_constant():
                    {"w": np.ones(2, np.float32), "v": np.zeros(2, np.float32)}, ["x"], ["y"])
     Engine(g, KernelRegistry().register(Probe())).run({"x": np.ones(2, np.float32), "v": np.ones(2, np.float32)})
     assert seen == {"x": False, "w": True, "v": False}
+
+
+def test_gqa_workspace_of_a_prompt_is_not_kept(monkeypatch):
+    """A decode step's workspace is the node's; a prompt's, as large as its keys and values, is
+    the call's own, and where it cannot be had the call goes without."""
+    import torch
+    from modelsharp_amd.decoder_kernels import HipGroupQueryAttentionKernel
+    from modelsharp_amd.graph import GraphNode
+    k = HipGroupQueryAttentionKernel()
+    node = GraphNode("GroupQueryAttention", "attn0", ["q"], ["out"], {})
+    assert k._workspace_for(node, 1, 0, "cpu") is None
+    step = k._workspace_for(node, 1, 1000, "cpu")
+    assert step.numel() * 4 >= 1000 and k._workspace_for(node, 8, 900, "cpu") is step
+    prompt = k._workspace_for(node, 200, 1 << 20, "cpu")
+    assert prompt.numel() * 4 >= 1 << 20 and list(k._workspace.values()) == [step]
+    assert k._workspace_for(node, 1, 1000, "cpu") is step
+
+    def full(*args, **kwargs):
+        raise torch.OutOfMemoryError("no memory")
+
+    monkeypatch.setattr(torch, "empty", full)
+    assert k._workspace_for(node, 200, 1 << 20, "cpu") is None
