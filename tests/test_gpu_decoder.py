@@ -454,6 +454,25 @@ def test_gqa_split_values_of_different_magnitude(gpu, D, exps):
     assert err.max() <= 3 * 2.0 ** -22
 
 
+# From 256 workgroups of 128 queries on, 128 queries share a workgroup (below, 64): head_dims
+# 96 and 128, ragged last blocks and chunks, a cached past, key ranges that end early, a window.
+SPLIT_WIDE_CASES = [
+    dict(seed=251, B=1, Sq=300, H=96, KH=8, D=128, past=37, cos_rows=340),
+    dict(seed=252, B=2, Sq=133, H=64, KH=4, D=128, past=64, seqlens=[70, 196], cos_rows=200),
+    dict(seed=253, B=1, Sq=258, H=96, KH=6, D=96, past=5, window=150, cos_rows=270),
+    dict(seed=254, B=4, Sq=140, H=32, KH=2, D=96, past=0, packed=True, cos_rows=140),
+]
+
+
+@pytest.mark.parametrize("case", SPLIT_WIDE_CASES, ids=lambda c: f"seed{c['seed']}")
+def test_gqa_split_wide_blocks(gpu, case):
+    d, q, k, v, pk, pv, sl, cos, sin = make_case(**case)
+    assert d.batch * d.num_heads * -(-d.q_seq // 128) >= 256
+    ref, rk, rv = oracle.gqa(d, q, k, v, pk, pv, sl, cos, sin)
+    check_gqa(*run_device_gqa(d, q, k, v, pk, pv, sl, cos, sin, capacity=d.past_seq + d.kv_seq + 5, workspace=True),
+              ref, rk, rv, f"split wide seed {case['seed']}")
+
+
 # Query blocks that the halves cannot carry (gqa_split_f32), every head_dim (64 from 192 keys on), both workgroup sizes
 # (128 queries from 256 workgroups on), ragged last blocks and chunks, a cached past, lengths
 # and windows that end inside a chunk with a special value.

@@ -545,8 +545,8 @@ def test_skinny_8bit(gpu, zp, K, ksw, bs):
 
 # mfma_block (the general formats with block sizes 16 to 512): block ends inside and across
 # its 64-k groups, a last group and a last block that are not full, rows and columns past its
-# tiles, and both launch shapes (64 x 128 tiles from one tile per CU on, else 32 x 64 with K
-# over four waves).
+# tiles; launches of 32 x 64 tiles with K over four waves (test_block_gemm_large_launch has the
+# others).
 BLOCK_OPS = [
     Op("b4_bs16_k24", 24, 70, 16, True),
     Op("b4_bs256", 1032, 129, 256, True),
@@ -715,3 +715,30 @@ def test_chunk_gemv_at_the_top_of_fp32(gpu, M, bits):
     y = w.gemm(a)
     assert np.array_equal(np.isnan(y), np.isnan(ref)) and np.array_equal(np.isinf(y), np.isinf(ref))
     w.close()
+
+
+# Launches of at least two 64 x 128 tiles per CU, where a workgroup takes whole K: every block
+# class, an odd number of 32-row fragments, ragged rows, columns and last blocks.
+@pytest.mark.parametrize("M,N", [(130, 21903), (97, 33001)])
+@pytest.mark.parametrize("fzp", [False, True], ids=["zp", "float_zp"])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("bs,K", [(16, 200), (32, 200), (64, 200), (128, 328), (512, 584)])
+def test_block_gemm_large_launch(gpu, bs, K, bits, fzp, M, N):
+    op = Op("block_large", K, N, bs, True, bits=bits)
+    b, s, z = workloads.make_weights(op, seed=K + M + bits)
+    zpf = float_zero_points(op, seed=bs + M) if fzp else None
+    z = None if fzp else z
+    a = workloads.make_activations(M, op.K, seed=M + 3, kind="rmsnorm")
+    w = native.NBitsWeights(b, s, zpf if fzp else z, op.N, op.K, op.bits, op.block_size)
+    cus = torch_cus()
+    whole = -(-M // 64) * -(-N // 128) >= 2 * cus
+    info = w.launch_info(M)
+    log(f"block large bs={bs} bits={bits} fzp={fzp} M={M} {info}")
+    assert info["kernel"] == "mfma_general" and info["lanes_per_row"] == (128 if whole else 64) and (whole or cus != 256)
+    check_against_oracle(w, a, b, s, z, zpf, op, f"block large bs={bs} bits={bits} M={M}")
+    w.close()
+
+
+def torch_cus():
+    import torch
+    return torch.cuda.get_device_properties(0).multi_processor_count
