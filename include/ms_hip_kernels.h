@@ -268,8 +268,12 @@ int ms_hip_qgemm_nbits(const float* a, const uint8_t* bq, const float* scales,
  * Bit for bit the reference's result (built without floating-point contraction).
  * bits 4 or 8, packed or default zero points (a handle with float zero points returns
  * MS_HIP_ERR_UNSUPPORTED, as the native seam declines them, NativeQuant.cs:87-89).
- * The workspace (M*ceil32(nb*bs) + 4*M*nb + 4*nb*ceil4(M) bytes, each 256-aligned)
- * is the handle's; it cannot grow under stream capture (MS_HIP_ERR_UNSUPPORTED). */
+ * The workspace is the handle's; it cannot grow under stream capture
+ * (MS_HIP_ERR_UNSUPPORTED). It holds the activation codes and their block scales: at
+ * M > 16 with 4-bit codes and a block size that is a multiple of 32 (up to 8800) as
+ * fp16 images, 2.25 bytes per activation of M rounded up to a multiple of 32, 64 or
+ * 128 rows and of K to one of 128; otherwise M*ceil32(nb*bs) + 4*M*nb bytes, each
+ * 256-aligned. */
 int ms_hip_nbits_gemm_dev_w4a8(void* handle, const float* dA, float* dY, int M, void* stream);
 int ms_hip_nbits_gemm_w4a8(void* handle, const float* a_host, float* y_host, int M);
 int ms_hip_qgemm_w4a8(const float* a, const uint8_t* bq, const float* scales,
@@ -399,10 +403,15 @@ typedef struct ms_hip_gqa_desc {
     int seqlens_len;
 } ms_hip_gqa_desc;
 int ms_hip_gqa_check(const ms_hip_gqa_desc* desc);
-/* Bytes of the optional workspace that lets few (batch, head, query) units over a long
- * history split their keys over several workgroups (0: no split for this shape). With
- * a smaller or NULL workspace ms_hip_gqa runs unsplit, or returns MS_HIP_ERR_UNSUPPORTED
- * when one workgroup cannot hold the history's scores. */
+/* Bytes of the optional workspace (0: this shape uses none). For few (batch, head,
+ * query) units over a long history it lets several workgroups share a unit's keys. For
+ * a prompt (more than 8 queries, head_dim 64, 96 or 128, 128 keys or more, 192 at
+ * head_dim 64) it holds the keys and values as fp16 halves, as many bytes as their fp32
+ * rows, for the matrix-core kernel of prompts; the workspace must then be 16-byte
+ * aligned. With a smaller, misaligned or NULL workspace ms_hip_gqa runs unsplit, a
+ * prompt on the slower fp32 kernels, or returns MS_HIP_ERR_UNSUPPORTED when one
+ * workgroup cannot hold the history's scores. The contents need not be kept from one
+ * call to the next; calls that may overlap need workspaces of their own. */
 int64_t ms_hip_gqa_workspace_size(const ms_hip_gqa_desc* desc);
 int ms_hip_gqa(const ms_hip_gqa_desc* desc, const float* dQ, const float* dK, const float* dV,
                const float* dPastK, const float* dPastV, const int32_t* dSeqlensK,

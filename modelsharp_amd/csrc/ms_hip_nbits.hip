@@ -14,10 +14,11 @@
 //     M <= 4, A panel fits LDS                                -> gemv_w8
 //   other formats (bits 8, float zero points, other block sizes or K), K and the block
 //   size multiples of 8:
-//     M <= 16                                                 -> gemv_general
-//     M >  16                                                 -> mfma_general (exact): with a
-//                                                                workspace and block sizes 16,
-//                                                                32, ..., 512 mfma_block's kernel
+//     M <= 16, block size a power of two of whole 16-byte
+//       chunks of codes                                       -> gemv_chunk (gemv_general.h)
+//     M <= 16 otherwise                                       -> gemv_general
+//     M >  16, block sizes 16, 32, ..., 512, a workspace      -> block_stage_a + mfma_block
+//     M >  16 otherwise                                       -> mfma_general (exact)
 //   anything else                                             -> generic
 // Declarations and reference citations: include/ms_hip_kernels.h.
 #include "../../include/ms_hip_kernels.h"
@@ -2940,7 +2941,7 @@ GqaPlan gqa_plan(const ms_hip_gqa_desc& d, int64_t ws_avail, bool split_ok = tru
             // 128 queries per workgroup while that still gives every CU one, else 64 (a block of
             // 64 halves a short launch's waves, and its idle CUs)
             const int64_t wg = (int64_t)d.batch * d.num_heads * ((d.q_seq + 127) / 128);
-            pl.split_waves = wg >= 256 ? 4 : 2;
+            pl.split_waves = wg >= device_cus() ? 4 : 2;
             pl.ws_bytes = ws;
             return pl;
         }
