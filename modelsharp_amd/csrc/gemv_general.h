@@ -20,51 +20,6 @@ namespace msnb {
 // Block sizes that are no power of two of whole 16-byte chunks (gemv_chunk_kernel below).
 constexpr int kGenRowsPerWg = 16;
 
-// Lane g's share of row n's sums: its 8-code groups.
-template <int M>
-__device__ __forceinline__ void gemv_general_sums(const RawLayout& L, const float* a, int n, int g, float (&acc)[M])
-{
-    const uint8_t* const brow = L.b + (int64_t)n * L.nb * L.blob;
-#pragma unroll
-    for (int m = 0; m < M; ++m) acc[m] = 0.0f;
-    const int groups = L.K >> 3;
-    for (int t = g; t < groups; t += 16) {
-        const int k0 = t << 3;
-        const int bk = k0 / L.bs, i0 = k0 - bk * L.bs;
-        const float s = L.scales[(int64_t)n * L.nb + bk];
-        const float zp = block_zp(L, n, bk);
-        const uint8_t* src = brow + (int64_t)bk * L.blob;
-        float w[8];
-        if (L.bits == 4) {
-            const uint32_t x = *reinterpret_cast<const uint32_t*>(src + (i0 >> 1));
-#pragma unroll
-            for (int i = 0; i < 8; ++i) w[i] = ((float)((x >> (4 * i)) & 0xFu) - zp) * s;
-        } else {
-            const uint2 x = *reinterpret_cast<const uint2*>(src + i0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                w[i] = ((float)((x.x >> (8 * i)) & 0xFFu) - zp) * s;
-                w[i + 4] = ((float)((x.y >> (8 * i)) & 0xFFu) - zp) * s;
-            }
-        }
-#pragma unroll
-        for (int m = 0; m < M; ++m) {
-            const float4 a0 = *reinterpret_cast<const float4*>(a + (int64_t)m * L.K + k0);
-            const float4 a1 = *reinterpret_cast<const float4*>(a + (int64_t)m * L.K + k0 + 4);
-            float t0 = acc[m];
-            t0 = __builtin_fmaf(a0.x, w[0], t0);
-            t0 = __builtin_fmaf(a0.y, w[1], t0);
-            t0 = __builtin_fmaf(a0.z, w[2], t0);
-            t0 = __builtin_fmaf(a0.w, w[3], t0);
-            t0 = __builtin_fmaf(a1.x, w[4], t0);
-            t0 = __builtin_fmaf(a1.y, w[5], t0);
-            t0 = __builtin_fmaf(a1.z, w[6], t0);
-            t0 = __builtin_fmaf(a1.w, w[7], t0);
-            acc[m] = t0;
-        }
-    }
-}
-
 template <int M>
 __global__ __launch_bounds__(256) void gemv_general_kernel(RawLayout L, const float* __restrict__ a,
                                                            float* __restrict__ y)
@@ -72,10 +27,48 @@ __global__ __launch_bounds__(256) void gemv_general_kernel(RawLayout L, const fl
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int g = lane & 15, r = lane >> 4;
     const int n = blockIdx.x * kGenRowsPerWg + wave * 4 + r;
+    const int64_t row_bytes = (int64_t)L.nb * L.blob;
     float acc[M];
 #pragma unroll
     for (int m = 0; m < M; ++m) acc[m] = 0.0f;
-    if (n < L.N) gemv_general_sums<M>(L, a, n, g, acc);
+    if (n < L.N) {
+        const int groups = L.K >> 3;
+        for (int t = g; t < groups; t += 16) {
+            const int k0 = t << 3;
+            const int bk = k0 / L.bs, i0 = k0 - bk * L.bs;
+            const float s = L.scales[(int64_t)n * L.nb + bk];
+            const float zp = block_zp(L, n, bk);
+            const uint8_t* src = L.b + (int64_t)n * row_bytes + (int64_t)bk * L.blob;
+            float w[8];
+            if (L.bits == 4) {
+                const uint32_t x = *reinterpret_cast<const uint32_t*>(src + (i0 >> 1));
+#pragma unroll
+                for (int i = 0; i < 8; ++i) w[i] = ((float)((x >> (4 * i)) & 0xFu) - zp) * s;
+            } else {
+                const uint2 x = *reinterpret_cast<const uint2*>(src + i0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    w[i] = ((float)((x.x >> (8 * i)) & 0xFFu) - zp) * s;
+                    w[i + 4] = ((float)((x.y >> (8 * i)) & 0xFFu) - zp) * s;
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const float4 a0 = *reinterpret_cast<const float4*>(a + (int64_t)m * L.K + k0);
+                const float4 a1 = *reinterpret_cast<const float4*>(a + (int64_t)m * L.K + k0 + 4);
+                float t0 = acc[m];
+                t0 = __builtin_fmaf(a0.x, w[0], t0);
+                t0 = __builtin_fmaf(a0.y, w[1], t0);
+                t0 = __builtin_fmaf(a0.z, w[2], t0);
+                t0 = __builtin_fmaf(a0.w, w[3], t0);
+                t0 = __builtin_fmaf(a1.x, w[4], t0);
+                t0 = __builtin_fmaf(a1.y, w[5], t0);
+                t0 = __builtin_fmaf(a1.z, w[6], t0);
+                t0 = __builtin_fmaf(a1.w, w[7], t0);
+                acc[m] = t0;
+            }
+        }
+    }
     // Every lane of the wave takes part in the scan (rows past N carry zeros).
 #pragma unroll
     for (int m = 0; m < M; ++m) acc[m] = group_sum_to_last<16>(acc[m]);
@@ -91,9 +84,9 @@ __global__ __launch_bounds__(256) void gemv_general_kernel(RawLayout L, const fl
 // point) in flight while the previous four compute; the activations come from LDS, float4 i of
 // chunk c of row m at (m F + i) C + c, so that the lanes of a row read consecutive words and the
 // rows of a wave the same ones. K passes in tiles of as many chunks as fit the panel.
-// A chunk's terms are added as sum a (q - zp), then acc += s times it, in fp32; a wave whose
-// sums come out infinite or NaN (activations above 7e35, times a code, pass the range that
-// their products with the scaled weights keep) takes them again as gemv_general_kernel does.
+// A chunk's terms are added as sum a (q - zp) 2^-9 (2^-12 at 8 bits), then acc += s 2^9 times it,
+// in fp32: powers of two change no rounding, and no finite activation passes the range of fp32
+// on the way to s times less (from 7e35 on it would; scales of 1 and more are taken as they are).
 // What bounds it is issue (3 + M VALU instructions per code) and the batches' round trips, not
 // the bytes. Float zero points, against gemv_general_kernel (whose 8-code groups each divided
 // by the block size and waited for their own loads): M=2, K=4096, N=11008, block 64: 26.1 ->
@@ -107,6 +100,7 @@ __global__ __launch_bounds__(512) void gemv_chunk_kernel(RawLayout L, const floa
                                                          int lcpb, int tile)
 {
     constexpr int F = B8 ? 4 : 8, U = 4;   // float4 of activations per chunk, chunks per batch
+    constexpr float kDown = B8 ? 4096.0f : 512.0f;   // above a chunk's sum of |code - zero point|
     extern __shared__ __attribute__((aligned(16))) float4 gen_panel[];
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     const int g = lane & 15, r = lane >> 4;
@@ -155,12 +149,15 @@ __global__ __launch_bounds__(512) void gemv_chunk_kernel(RawLayout L, const floa
                 for (int m = 0; m < M; ++m) t[m] = 0.0f;
                 const uint32_t q[4] = {w.q[u].x, w.q[u].y, w.q[u].z, w.q[u].w};
                 const float4* const pa = gen_panel + (c - t0);
+                const bool small = fabsf(w.s[u]) < 1.0f;
+                const float k = small ? 1.0f / kDown : 1.0f, zk = -(w.z[u] * k), sk = small ? w.s[u] * kDown : w.s[u];
 #pragma unroll
                 for (int i = 0; i < F; ++i) {   // codes 4 i .. 4 i + 3 of the chunk
                     float d[4];
 #pragma unroll
                     for (int b = 0; b < 4; ++b)
-                        d[b] = (float)(B8 ? (q[i] >> (8 * b)) & 0xFFu : (q[i >> 1] >> (16 * (i & 1) + 4 * b)) & 0xFu) - w.z[u];
+                        d[b] = __builtin_fmaf(
+                            (float)(B8 ? (q[i] >> (8 * b)) & 0xFFu : (q[i >> 1] >> (16 * (i & 1) + 4 * b)) & 0xFu), k, zk);
 #pragma unroll
                     for (int m = 0; m < M; ++m) {
                         const float4 v = pa[(m * F + i) * tile];
@@ -171,22 +168,13 @@ __global__ __launch_bounds__(512) void gemv_chunk_kernel(RawLayout L, const floa
                     }
                 }
 #pragma unroll
-                for (int m = 0; m < M; ++m) acc[m] = __builtin_fmaf(w.s[u], t[m], acc[m]);
+                for (int m = 0; m < M; ++m) acc[m] = __builtin_fmaf(sk, t[m], acc[m]);
             }
             w = nx;
         }
     }
-    bool finite = true;
 #pragma unroll
-    for (int m = 0; m < M; ++m) {
-        acc[m] = group_sum_to_last<16>(acc[m]);
-        finite = finite && fabsf(acc[m]) <= 3.402823466e38f;
-    }
-    if (!__all(finite || g != 15)) {
-        gemv_general_sums<M>(L, a, (int)nr, g, acc);
-#pragma unroll
-        for (int m = 0; m < M; ++m) acc[m] = group_sum_to_last<16>(acc[m]);
-    }
+    for (int m = 0; m < M; ++m) acc[m] = group_sum_to_last<16>(acc[m]);
     if (g == 15 && live) {
 #pragma unroll
         for (int m = 0; m < M; ++m) y[(int64_t)m * L.N + n] = acc[m];
