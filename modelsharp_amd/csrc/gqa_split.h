@@ -29,11 +29,13 @@
 //     LDS: a K and a V chunk per group (1 KB * D in all), filled by buffer->LDS loads that
 //     are issued one phase before they are waited for. One barrier per phase.
 //
-// 28 / 4 heads of 128, 2048 queries and keys: 126 us with the conversion (14 us of it),
-// 239 TFLOP/s of causal work, where gqa_flash_kernel took 637; its error against 64 bits is
-// 2.7e-7 (4.5e-7). 32 / 8 heads of 96 over 1000 tokens: 60 us, 1111 before
-// (gqa_attention_kernel). The MFMAs are busy 31% of the time, the VALU (630 instructions per
-// wave and chunk) as much: what is left is the waits at each phase's barrier.
+// 28 / 4 heads of 128, 2048 queries and keys: 127 us with the conversion (13 us of it),
+// 237 TFLOP/s of causal work, where gqa_flash_kernel took 637; its error against 64 bits is
+// 2.3e-7 (4.5e-7). 32 / 8 heads of 96 over 1000 tokens: 60 us, 1111 before
+// (gqa_attention_kernel); 1196 tokens, 16 / 2 heads of 128: 71 us. Following V's exponents
+// chunk by chunk costs 0.5 us of the 127 (1 of the 71). The MFMAs are busy 31% of the time, the
+// VALU (630 instructions per wave and chunk) as much: what is left is the waits at each phase's
+// barrier.
 // What the halves cannot carry (an infinity, a NaN, |q| or |k| >= 2^50, key or value rows of a
 // chunk more than 2^12 apart: a row seen by queries that do not see the larger one would lose
 // its low bits; chunks of V more than 2^60 apart) sends the query blocks that meet it to

@@ -14,8 +14,8 @@
 // instructions per 8 codes of a lane and 16 or 32 per 32 x 32 outputs and block. A wave's
 // tile of 32 rows of A x 64 weight rows balances the two at block size 64; each A operand
 // read from LDS feeds 4 MFMAs. Float zero points, against mfma_general: M=512, K=N=4096,
-// block 64: 236 -> 98 us (the MFMAs' time is 28: what is left is the waits at a barrier per
-// 64 k); M=32: 222 -> 34 us; M=1000, K=2048, N=4000, block 16: 157 -> 85 us. 8-bit codes, M=128,
+// block 64: 236 -> 94 us (98 without the loads' wait states; the MFMAs' time is 28: what is
+// left is the waits at a barrier per 64 k); M=32: 222 -> 34 us; M=1000, K=2048, N=4000, block 16: 157 -> 85 us. 8-bit codes, M=128,
 // K=N=4096, block 32: 232 -> 40 us. Error against 64 bits 1e-7 to 2e-7 (3e-7 to 1e-6).
 //
 //   block_stage_a_kernel  one workgroup per row: e[m], the halves in MFMA operand order, one

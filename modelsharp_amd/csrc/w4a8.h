@@ -174,7 +174,7 @@ __global__ __launch_bounds__(256) void gemv_w4a8_kernel(RawLayout L, W4a8Args A,
 //     block scales behind the codes, double-buffered through buffer->LDS loads issued a
 //     group ahead: one barrier per 128 k, no bank conflicts.
 // Workgroups of 4 waves take 64 weight rows; NF (2, 4 or 8) by launch size.
-// M=256, K=4096, N=11008, bs=32: 156 -> 80 us; M=128, K=11008, N=4096, bs=128: 254 -> 88 us;
+// M=256, K=4096, N=11008, bs=32: 156 -> 79 us; M=128, K=11008, N=4096, bs=128: 254 -> 88 us;
 // M=17, K=4096, N=4096: 132 -> 50 us (against an int8 MFMA, a barrier per 32 codes and loads
 // that were not ahead). What is left above the VALU's time is the wait for each group's loads.
 constexpr int kW8BN = 64;
