@@ -454,6 +454,23 @@ def test_gqa_split_values_of_different_magnitude(gpu, D, exps):
     assert err.max() <= 3 * 2.0 ** -22
 
 
+@pytest.mark.parametrize("peak", [2, 8])
+@pytest.mark.parametrize("D", [64, 96, 128])
+def test_gqa_split_small_weights(gpu, D, peak):
+    """Peaked softmax rows over values of which the first 64 are 2^11 smaller than the rest:
+    small weights keep their bits beside the block's larger values. Queries and keys of few
+    bits, so that no score is rounded before the softmax; the bound of the test above
+    (measured 5e-7; 2e-6 to 5e-6 where V's exponent is folded into the weights)."""
+    d, q, k, v, *_ = make_case(233, B=1, Sq=256, H=4, KH=2, D=D, past=0, rotary=False, cos_rows=8)
+    q, k = (np.round(q * 2) / 2 * peak).astype(np.float32), (np.round(k * 2) / 2).astype(np.float32)
+    v[:, :64] *= np.float32(2.0 ** -11)
+    out, _, _ = run_device_gqa(d, q, k, v, None, None, None, None, None, workspace=True)
+    ref = np.asarray(gqa_f64(d, q, k, v, None, None, None, None, None)[0]).reshape(-1, D)
+    err = np.linalg.norm(out.reshape(-1, D) - ref, axis=-1) / np.linalg.norm(ref, axis=-1)
+    log(f"split D={D} peak {peak}: largest row error {err.max():.2e}")
+    assert err.max() <= 3 * 2.0 ** -22
+
+
 # From 256 workgroups of 128 queries on, 128 queries share a workgroup (below, 64): head_dims
 # 96 and 128, ragged last blocks and chunks, a cached past, key ranges that end early, a window.
 SPLIT_WIDE_CASES = [
