@@ -84,9 +84,10 @@ __global__ __launch_bounds__(256) void gemv_general_kernel(RawLayout L, const fl
 // point) in flight while the previous four compute; the activations come from LDS, float4 i of
 // chunk c of row m at (m F + i) C + c, so that the lanes of a row read consecutive words and the
 // rows of a wave the same ones. K passes in tiles of as many chunks as fit the panel.
-// A chunk's terms are added as sum a (q - zp) 2^-9 (2^-12 at 8 bits), then acc += s 2^9 times it,
-// in fp32: powers of two change no rounding, and no finite activation passes the range of fp32
-// on the way to s times less (from 7e35 on it would; scales of 1 and more are taken as they are).
+// A chunk's terms are added as sum a (q - zp) 2^-9 (2^-12 at 8 bits), then acc += s times it, in
+// fp32, and the result is taken back: no finite activation passes the range of fp32 on the way to
+// s times less (without it from 7e35 on), and no rounding changes in sums above 1e-34. It costs a
+// multiplication per chunk, 0 to 0.6%.
 // What bounds it is issue (3 + M VALU instructions per code) and the batches' round trips, not
 // the bytes. Float zero points, against gemv_general_kernel (whose 8-code groups each divided
 // by the block size and waited for their own loads): M=2, K=4096, N=11008, block 64: 26.1 ->
@@ -149,15 +150,14 @@ __global__ __launch_bounds__(512) void gemv_chunk_kernel(RawLayout L, const floa
                 for (int m = 0; m < M; ++m) t[m] = 0.0f;
                 const uint32_t q[4] = {w.q[u].x, w.q[u].y, w.q[u].z, w.q[u].w};
                 const float4* const pa = gen_panel + (c - t0);
-                const bool small = fabsf(w.s[u]) < 1.0f;
-                const float k = small ? 1.0f / kDown : 1.0f, zk = -(w.z[u] * k), sk = small ? w.s[u] * kDown : w.s[u];
+                const float zk = -(w.z[u] * (1.0f / kDown));
 #pragma unroll
                 for (int i = 0; i < F; ++i) {   // codes 4 i .. 4 i + 3 of the chunk
                     float d[4];
 #pragma unroll
                     for (int b = 0; b < 4; ++b)
                         d[b] = __builtin_fmaf(
-                            (float)(B8 ? (q[i] >> (8 * b)) & 0xFFu : (q[i >> 1] >> (16 * (i & 1) + 4 * b)) & 0xFu), k, zk);
+                            (float)(B8 ? (q[i] >> (8 * b)) & 0xFFu : (q[i >> 1] >> (16 * (i & 1) + 4 * b)) & 0xFu), 1.0f / kDown, zk);
 #pragma unroll
                     for (int m = 0; m < M; ++m) {
                         const float4 v = pa[(m * F + i) * tile];
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(512) void gemv_chunk_kernel(RawLayout L, const floa
                     }
                 }
 #pragma unroll
-                for (int m = 0; m < M; ++m) acc[m] = __builtin_fmaf(sk, t[m], acc[m]);
+                for (int m = 0; m < M; ++m) acc[m] = __builtin_fmaf(w.s[u], t[m], acc[m]);
             }
             w = nx;
         }
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(512) void gemv_chunk_kernel(RawLayout L, const floa
     for (int m = 0; m < M; ++m) acc[m] = group_sum_to_last<16>(acc[m]);
     if (g == 15 && live) {
 #pragma unroll
-        for (int m = 0; m < M; ++m) y[(int64_t)m * L.N + n] = acc[m];
+        for (int m = 0; m < M; ++m) y[(int64_t)m * L.N + n] = acc[m] * kDown;
     }
 }
 

@@ -709,6 +709,8 @@ def test_chunk_gemv_at_the_top_of_fp32(gpu, M, bits):
     w = native.NBitsWeights(b, s, zpf, op.N, op.K, op.bits, op.block_size)
     kernel, _ = check_against_oracle(w, a, b, s, None, zpf, op, f"chunk bits={bits} M={M} at {top}")
     assert kernel == "gemv_general"
+    low = workloads.make_activations(M, op.K, seed=M) * np.float32(1e-33)   # and near its bottom
+    check_against_oracle(w, low, b, s, None, zpf, op, f"chunk bits={bits} M={M} at 1e-33")
     a[0, 3], a[-1, 7] = np.inf, np.nan
     with np.errstate(all="ignore"):
         ref = oracle.matmul_nbits(a, b, s, None, op.N, op.K, op.bits, op.block_size, zp_float=zpf)
